@@ -49,9 +49,9 @@ template <typename T>
 __global__ __launch_bounds__(kThreads) void k_init(const SysDev* __restrict__ sys, const int3* __restrict__ work) {
     using C = cplx_t<T>;
     VEC_PROLOGUE
-    const C* b = (const C*)d.b;
-    C *x = (C*)d.x, *r = (C*)d.r, *r0 = (C*)d.r0, *p = (C*)d.p, *v = (C*)d.v;
-    C *y = (C*)d.y, *zz = (C*)d.z;  // the preconditioned operands (alias p, s without a preconditioner)
+    const C* b = glob((const C*)d.b);
+    C *x = glob((C*)d.x), *r = glob((C*)d.r), *r0 = glob((C*)d.r0), *p = glob((C*)d.p), *v = glob((C*)d.v);
+    C *y = glob((C*)d.y), *zz = glob((C*)d.z);  // the preconditioned operands (alias p, s without a preconditioner)
     const bool x0_b = (d.flags & MPA_SOLVE_REF_LOOP) != 0;  // r = b - A b is formed by the restart kernels
     double2 acc[1] = {make_double2(0, 0)};
     for (int i = g * kThreads + threadIdx.x; i < n; i += stride) {
@@ -71,7 +71,7 @@ __global__ __launch_bounds__(kThreads) void k_init(const SysDev* __restrict__ sy
         acc[0].x += bd.x * bd.x + bd.y * bd.y;
     }
     block_sum<1>(acc);
-    if (threadIdx.x == 0) d.part[((size_t)s * d.G + g) * kSlots + 3] = acc[0];
+    if (threadIdx.x == 0) glob(d.part)[((size_t)s * d.G + g) * kSlots + 3] = acc[0];
 }
 
 __global__ __launch_bounds__(kThreads) void k_init_scalars(const SysDev* __restrict__ sys, const int2* __restrict__ cw) {
@@ -80,7 +80,7 @@ __global__ __launch_bounds__(kThreads) void k_init_scalars(const SysDev* __restr
     const int s = c2.y;
     const double2 bb = reduce_partials(d.part, d.G, s, 3);
     if (threadIdx.x == 0) {
-        Scal& c = d.scal[s];
+        Scal& c = glob(d.scal)[s];
         const bool ref = (d.flags & MPA_SOLVE_REF_LOOP) != 0;
         c.rho = c.alpha = c.w = make_double2(1, 0);
         c.alpha_next = c.w_next = make_double2(1, 0);
@@ -116,11 +116,11 @@ template <typename T>
 __global__ __launch_bounds__(kThreads) void k_update_p(const SysDev* __restrict__ sys, const int3* __restrict__ work) {
     using C = cplx_t<T>;
     VEC_PROLOGUE
-    const Scal& c = d.scal[s];
+    const Scal& c = glob(d.scal)[s];
     if (c.done || c.restart_pending) return;
     const double2 beta = cmul(cdiv(c.rho_next, c.rho), cdiv(c.alpha, c.w));
     const C bt = from_d<T>(beta), wt = from_d<T>(c.w);
-    C *p = (C*)d.p, *r = (C*)d.r, *v = (C*)d.v;
+    C *p = glob((C*)d.p), *r = glob((C*)d.r), *v = glob((C*)d.v);
     for (int i = g * kThreads + threadIdx.x; i < n; i += stride) {
         const size_t k = base + i;
         p[k] = cadd(r[k], cmul(bt, csub(p[k], cmul(wt, v[k]))));
@@ -138,11 +138,11 @@ __global__ __launch_bounds__(kThreads) void k_precond(const SysDev* __restrict__
     using C = cplx_t<T>;
     VEC_PROLOGUE
     if (!d.minv) return;
-    const Scal& c = d.scal[s];
+    const Scal& c = glob(d.scal)[s];
     if (c.done || c.restart_pending) return;
-    const C* src = (const C*)(which ? d.s : d.p) + base;
-    C* dst = (C*)(which ? d.z : d.y) + base;
-    const C* M = (const C*)d.minv;
+    const C* src = glob((const C*)(which ? d.s : d.p)) + base;
+    C* dst = glob((C*)(which ? d.z : d.y)) + base;
+    const C* M = glob((const C*)d.minv);
     const int bs = d.bs;
     for (int i = g * kThreads + threadIdx.x; i < n; i += stride) {
         const C* row = M + (size_t)i * bs;
@@ -158,12 +158,12 @@ template <typename T>
 __global__ __launch_bounds__(kThreads) void k_dot_r0v(const SysDev* __restrict__ sys, const int3* __restrict__ work) {
     using C = cplx_t<T>;
     VEC_PROLOGUE
-    if (d.scal[s].done || d.scal[s].restart_pending) return;
-    const C *r0 = (const C*)d.r0, *v = (const C*)d.v;
+    if (glob(d.scal)[s].done || glob(d.scal)[s].restart_pending) return;
+    const C *r0 = glob((const C*)d.r0), *v = glob((const C*)d.v);
     double2 acc[1] = {make_double2(0, 0)};
     for (int i = g * kThreads + threadIdx.x; i < n; i += stride) acc[0] = cadd(acc[0], cmulc(to_d(r0[base + i]), to_d(v[base + i])));
     block_sum<1>(acc);
-    if (threadIdx.x == 0) d.part[((size_t)s * d.G + g) * kSlots + 0] = acc[0];
+    if (threadIdx.x == 0) glob(d.part)[((size_t)s * d.G + g) * kSlots + 0] = acc[0];
 }
 
 // alpha = rho / <r0, v>; s = r - alpha v
@@ -171,13 +171,13 @@ template <typename T>
 __global__ __launch_bounds__(kThreads) void k_update_s(const SysDev* __restrict__ sys, const int3* __restrict__ work) {
     using C = cplx_t<T>;
     VEC_PROLOGUE
-    if (d.scal[s].done || d.scal[s].restart_pending) return;
+    if (glob(d.scal)[s].done || glob(d.scal)[s].restart_pending) return;
     const double2 dv = reduce_partials(d.part, d.G, s, 0);
-    const double2 alpha = cdiv(d.scal[s].rho_next, dv);
+    const double2 alpha = cdiv(glob(d.scal)[s].rho_next, dv);
     const C at = from_d<T>(alpha);
-    C *sv = (C*)d.s, *r = (C*)d.r, *v = (C*)d.v;
+    C *sv = glob((C*)d.s), *r = glob((C*)d.r), *v = glob((C*)d.v);
     for (int i = g * kThreads + threadIdx.x; i < n; i += stride) sv[base + i] = csub(r[base + i], cmul(at, v[base + i]));
-    if (g == 0 && threadIdx.x == 0) d.scal[s].alpha_next = alpha;
+    if (g == 0 && threadIdx.x == 0) glob(d.scal)[s].alpha_next = alpha;
 }
 
 // partials <t, s>, <t, t>
@@ -185,8 +185,8 @@ template <typename T>
 __global__ __launch_bounds__(kThreads) void k_dot_ts(const SysDev* __restrict__ sys, const int3* __restrict__ work) {
     using C = cplx_t<T>;
     VEC_PROLOGUE
-    if (d.scal[s].done || d.scal[s].restart_pending) return;
-    const C *tv = (const C*)d.t, *sv = (const C*)d.s;
+    if (glob(d.scal)[s].done || glob(d.scal)[s].restart_pending) return;
+    const C *tv = glob((const C*)d.t), *sv = glob((const C*)d.s);
     double2 acc[2] = {make_double2(0, 0), make_double2(0, 0)};
     for (int i = g * kThreads + threadIdx.x; i < n; i += stride) {
         const double2 t = to_d(tv[base + i]);
@@ -195,8 +195,8 @@ __global__ __launch_bounds__(kThreads) void k_dot_ts(const SysDev* __restrict__ 
     }
     block_sum<2>(acc);
     if (threadIdx.x == 0) {
-        d.part[((size_t)s * d.G + g) * kSlots + 1] = acc[0];
-        d.part[((size_t)s * d.G + g) * kSlots + 2] = acc[1];
+        glob(d.part)[((size_t)s * d.G + g) * kSlots + 1] = acc[0];
+        glob(d.part)[((size_t)s * d.G + g) * kSlots + 2] = acc[1];
     }
 }
 
@@ -205,13 +205,13 @@ template <typename T>
 __global__ __launch_bounds__(kThreads) void k_update_xr(const SysDev* __restrict__ sys, const int3* __restrict__ work) {
     using C = cplx_t<T>;
     VEC_PROLOGUE
-    if (d.scal[s].done || d.scal[s].restart_pending) return;
+    if (glob(d.scal)[s].done || glob(d.scal)[s].restart_pending) return;
     const double2 ts = reduce_partials(d.part, d.G, s, 1);
     const double2 tt = reduce_partials(d.part, d.G, s, 2);
     const double2 om = tt.x > 0 ? cscale(ts, 1.0 / tt.x) : make_double2(0, 0);
-    const C at = from_d<T>(d.scal[s].alpha_next), wt = from_d<T>(om);
+    const C at = from_d<T>(glob(d.scal)[s].alpha_next), wt = from_d<T>(om);
     // y, z alias p, s without a preconditioner
-    C *x = (C*)d.x, *y = (C*)d.y, *z = (C*)d.z, *sv = (C*)d.s, *tv = (C*)d.t, *r = (C*)d.r, *r0 = (C*)d.r0;
+    C *x = glob((C*)d.x), *y = glob((C*)d.y), *z = glob((C*)d.z), *sv = glob((C*)d.s), *tv = glob((C*)d.t), *r = glob((C*)d.r), *r0 = glob((C*)d.r0);
     const bool pc = d.minv != nullptr;
     double2 acc[2] = {make_double2(0, 0), make_double2(0, 0)};
     for (int i = g * kThreads + threadIdx.x; i < n; i += stride) {
@@ -226,10 +226,10 @@ __global__ __launch_bounds__(kThreads) void k_update_xr(const SysDev* __restrict
     }
     block_sum<2>(acc);
     if (threadIdx.x == 0) {
-        d.part[((size_t)s * d.G + g) * kSlots + 3] = acc[0];
-        d.part[((size_t)s * d.G + g) * kSlots + 4] = acc[1];
+        glob(d.part)[((size_t)s * d.G + g) * kSlots + 3] = acc[0];
+        glob(d.part)[((size_t)s * d.G + g) * kSlots + 4] = acc[1];
     }
-    if (g == 0 && threadIdx.x == 0) d.scal[s].w_next = om;
+    if (g == 0 && threadIdx.x == 0) glob(d.scal)[s].w_next = om;
 }
 
 // commit the iteration's scalars; convergence, maxiter and restart checks
@@ -237,7 +237,7 @@ __global__ __launch_bounds__(kThreads) void k_commit(const SysDev* __restrict__ 
     const int2 c2 = cw[blockIdx.x];
     const SysDev& d = sys[c2.x];
     const int s = c2.y;
-    Scal& c = d.scal[s];
+    Scal& c = glob(d.scal)[s];
     if (c.done || c.restart_pending) return;
     const double2 rr = reduce_partials(d.part, d.G, s, 3);
     const double2 r0r = reduce_partials(d.part, d.G, s, 4);
@@ -269,9 +269,9 @@ template <typename T>
 __global__ __launch_bounds__(kThreads) void k_restart(const SysDev* __restrict__ sys, const int3* __restrict__ work) {
     using C = cplx_t<T>;
     VEC_PROLOGUE
-    if (!d.scal[s].restart_pending) return;
-    const C *b = (const C*)d.b, *tv = (const C*)d.t;
-    C *r = (C*)d.r, *r0 = (C*)d.r0;
+    if (!glob(d.scal)[s].restart_pending) return;
+    const C *b = glob((const C*)d.b), *tv = glob((const C*)d.t);
+    C *r = glob((C*)d.r), *r0 = glob((C*)d.r0);
     double2 acc[1] = {make_double2(0, 0)};
     for (int i = g * kThreads + threadIdx.x; i < n; i += stride) {
         const size_t k = base + i;
@@ -282,17 +282,17 @@ __global__ __launch_bounds__(kThreads) void k_restart(const SysDev* __restrict__
         acc[0].x += rd.x * rd.x + rd.y * rd.y;
     }
     block_sum<1>(acc);
-    if (threadIdx.x == 0) d.part[((size_t)s * d.G + g) * kSlots + 3] = acc[0];
+    if (threadIdx.x == 0) glob(d.part)[((size_t)s * d.G + g) * kSlots + 3] = acc[0];
 }
 
 __global__ __launch_bounds__(kThreads) void k_restart_commit(const SysDev* __restrict__ sys, const int2* __restrict__ cw) {
     const int2 c2 = cw[blockIdx.x];
     const SysDev& d = sys[c2.x];
     const int s = c2.y;
-    if (!d.scal[s].restart_pending) return;
+    if (!glob(d.scal)[s].restart_pending) return;
     const double2 rr = reduce_partials(d.part, d.G, s, 3);
     if (threadIdx.x == 0) {
-        Scal& c = d.scal[s];
+        Scal& c = glob(d.scal)[s];
         // Eigen: rho = r0_sqnorm = ||r||^2 replaces this iteration's rho; the
         // committed rho stays as rho_old for beta = (rho/rho_old)(alpha/w).
         c.r0_sq = rr.x;
@@ -317,7 +317,7 @@ __global__ __launch_bounds__(kThreads) void k_restart_commit(const SysDev* __res
 __global__ __launch_bounds__(64) void k_gather_scalars(const SysDev* __restrict__ sys, const int2* __restrict__ cw,
                                                         int count, Scal* __restrict__ out) {
     const int k = blockIdx.x * 64 + threadIdx.x;
-    if (k < count) out[k] = sys[cw[k].x].scal[cw[k].y];
+    if (k < count) out[k] = glob(sys[cw[k].x].scal)[cw[k].y];
 }
 
 // ---- host side ---------------------------------------------------------------------

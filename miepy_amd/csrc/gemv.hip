@@ -49,8 +49,9 @@ __device__ inline void chunk_fma(float& ar, float& ai, fvec4 a, fvec4 x) {
 }
 
 __device__ inline bool all_done(const SysDev& d) {
+    const Scal* scal = glob(d.scal);
     for (int s = 0; s < d.S; s++)
-        if (!d.scal[s].done) return false;
+        if (!scal[s].done) return false;
     return true;
 }
 
@@ -65,7 +66,7 @@ __device__ inline void gemv_rows(const MvDev& J, int rb) {
     const int row0 = (rb * 4 + w) * R;
     if (row0 >= n) return;
     const int nv = n / C;  // 16-byte chunks per row (n is even)
-    const T* A = (const T*)J.A;
+    const T* A = glob((const T*)J.A);
     const V* Ar[R];
 #pragma unroll
     for (int r = 0; r < R; r++) Ar[r] = (const V*)(A + (size_t)2 * n * min(row0 + r, n - 1));
@@ -77,7 +78,7 @@ __device__ inline void gemv_rows(const MvDev& J, int rb) {
             for (int s = 0; s < SG; s++) ar[r][s] = ai[r][s] = 0;
         const V* xs[SG];
 #pragma unroll
-        for (int s = 0; s < SG; s++) xs[s] = (const V*)((const T*)J.x + (size_t)2 * n * min(s0 + s, J.S - 1));
+        for (int s = 0; s < SG; s++) xs[s] = (const V*)(glob((const T*)J.x) + (size_t)2 * n * min(s0 + s, J.S - 1));
         int c = lane;
         for (; c + 64 * (U - 1) < nv; c += 64 * U) {
             V xv[SG][U];
@@ -121,8 +122,8 @@ __device__ inline void gemv_rows(const MvDev& J, int rb) {
                 if (lane == 0 && row < n && s0 + s < J.S) {
                     const size_t o = (size_t)(s0 + s) * n + row;
                     cplx_t<T> yv = cmake<T>(re, im);
-                    if (J.add_identity) yv = cadd(yv, ((const cplx_t<T>*)J.x)[o]);
-                    ((cplx_t<T>*)J.y)[o] = yv;
+                    if (J.add_identity) yv = cadd(yv, glob((const cplx_t<T>*)J.x)[o]);
+                    glob((cplx_t<T>*)J.y)[o] = yv;
                 }
             }
     }
@@ -175,8 +176,8 @@ __device__ inline void gemm_rows_c64(const MvDev& J, int rb) {
     const int n = J.n;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int h = lane >> 5, col = lane & 31, s_of = col >> 1, part = col & 1;
-    const float2* A = (const float2*)J.A;
-    const float2* X = (const float2*)J.x;
+    const float2* A = glob((const float2*)J.A);
+    const float2* X = glob((const float2*)J.x);
     const int nkb = (n + kGemmKB - 1) / kGemmKB;
     // global -> register staging of one K step: thread loads 8 chunks of 16 B
     // (chunk id = it * 256 + tid: 16 chunks per row, a wave covers 4 full rows)
@@ -247,8 +248,8 @@ __device__ inline void gemm_rows_c64(const MvDev& J, int rb) {
             if (r < n && s < J.S && s_of < kGemmS) {
                 const size_t o = 2 * ((size_t)s * n + r) + part;
                 float v = acc[i];
-                if (J.add_identity) v += ((const float*)J.x)[o];
-                ((float*)J.y)[o] = v;
+                if (J.add_identity) v += glob((const float*)J.x)[o];
+                glob((float*)J.y)[o] = v;
             }
         }
     }
@@ -271,8 +272,8 @@ __device__ inline void gemm_rows_c64_s8(const MvDev& J, int rb) {
     const int n = J.n;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int g = lane >> 4, col = lane & 15, s_of = col >> 1, part = col & 1;
-    const float2* A = (const float2*)J.A;
-    const float2* X = (const float2*)J.x;
+    const float2* A = glob((const float2*)J.A);
+    const float2* X = glob((const float2*)J.x);
     const int nkb = (n + kGemmKB - 1) / kGemmKB;
     for (int s0 = 0; s0 < J.S; s0 += kGemmS8) {
         // A: 128 rows x 16 chunks of 16 B, 8 per thread (a wave covers 4 full rows per it)
@@ -338,8 +339,8 @@ __device__ inline void gemm_rows_c64_s8(const MvDev& J, int rb) {
                 if (r < n && s < J.S) {
                     const size_t o = 2 * ((size_t)s * n + r) + part;
                     float v = t ? acc1[i] : acc0[i];
-                    if (J.add_identity) v += ((const float*)J.x)[o];
-                    ((float*)J.y)[o] = v;
+                    if (J.add_identity) v += glob((const float*)J.x)[o];
+                    glob((float*)J.y)[o] = v;
                 }
             }
     }
@@ -357,8 +358,8 @@ __device__ inline void gemm_rows_c128(const MvDev& J, int rb) {
     const int n = J.n;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int g = lane >> 4, col = lane & 15, s_of = col >> 1, part = col & 1;
-    const double2* A = (const double2*)J.A;
-    const double2* X = (const double2*)J.x;
+    const double2* A = glob((const double2*)J.A);
+    const double2* X = glob((const double2*)J.x);
     const int nkb = (n + kGemmKB - 1) / kGemmKB;
     // 64 rows x 32 complex = 2048 chunks of 16 B (one complex each): thread loads 8
     // (chunk id = it * 256 + tid: 32 chunks per row, a wave covers 2 full rows)
@@ -436,8 +437,8 @@ __device__ inline void gemm_rows_c128(const MvDev& J, int rb) {
                 if (r < n && s < J.S) {
                     const size_t o = 2 * ((size_t)s * n + r) + part;
                     double v = c ? acc1[i] : acc0[i];
-                    if (J.add_identity) v += ((const double*)J.x)[o];
-                    ((double*)J.y)[o] = v;
+                    if (J.add_identity) v += glob((const double*)J.x)[o];
+                    glob((double*)J.y)[o] = v;
                 }
             }
         }

@@ -53,13 +53,13 @@ __global__ __launch_bounds__(kThreads) void k_ref_start(const RefDev* __restrict
     REF_PROLOGUE
     double2 acc[1] = {make_double2(0, 0)};
     for (int i = g * kThreads + threadIdx.x; i < n; i += stride) {
-        const double2 bv = d.b[base + i];
-        d.r[base + i] = bv;
-        d.x[base + i] = make_double2(0, 0);
+        const double2 bv = glob(d.b)[base + i];
+        glob(d.r)[base + i] = bv;
+        glob(d.x)[base + i] = make_double2(0, 0);
         acc[0].x += bv.x * bv.x + bv.y * bv.y;
     }
     block_sum<1>(acc);
-    if (threadIdx.x == 0) d.part[(size_t)s * d.G + g] = acc[0];
+    if (threadIdx.x == 0) glob(d.part)[(size_t)s * d.G + g] = acc[0];
 }
 
 // norms[s] = sum of the partials (fixed order), one block per (system, RHS)
@@ -69,14 +69,14 @@ __global__ __launch_bounds__(kThreads) void k_ref_norms(const RefDev* __restrict
     const int s = c2.y;
     __shared__ double red[kThreads];
     double a = 0;
-    for (int g = threadIdx.x; g < d.G; g += kThreads) a += d.part[(size_t)s * d.G + g].x;
+    for (int g = threadIdx.x; g < d.G; g += kThreads) a += glob(d.part)[(size_t)s * d.G + g].x;
     red[threadIdx.x] = a;
     __syncthreads();
     for (int w = kThreads / 2; w > 0; w >>= 1) {
         if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
         __syncthreads();
     }
-    if (threadIdx.x == 0) d.norms[s] = red[0];
+    if (threadIdx.x == 0) glob(d.norms)[s] = red[0];
 }
 
 // Per-RHS values between the systems' records and one flat array in
@@ -91,34 +91,34 @@ __global__ __launch_bounds__(kThreads) void k_ref_flat(const RefDev* __restrict_
     const int2 c2 = cw[k];
     const RefDev& d = sys[c2.x];
     if (mode == 0) {
-        flat[k] = d.norms[c2.y];
+        flat[k] = glob(d.norms)[c2.y];
     } else {
-        if (mode == 1) d.scale[c2.y] = flat[total + k];
-        d.unscale[c2.y] = flat[2 * total + k];
+        if (mode == 1) glob(d.scale)[c2.y] = flat[total + k];
+        glob(d.unscale)[c2.y] = flat[2 * total + k];
     }
 }
 
 // r32 = r * scale, rounded to complex64
 __global__ __launch_bounds__(kThreads) void k_ref_to32(const RefDev* __restrict__ sys, const int3* __restrict__ work) {
     REF_PROLOGUE
-    const double f = d.scale[s];
+    const double f = glob(d.scale)[s];
     for (int i = g * kThreads + threadIdx.x; i < n; i += stride) {
-        const double2 z = d.r[base + i];
-        d.r32[base + i] = make_float2((float)(z.x * f), (float)(z.y * f));
+        const double2 z = glob(d.r)[base + i];
+        glob(d.r32)[base + i] = make_float2((float)(z.x * f), (float)(z.y * f));
     }
 }
 
 // x += d32 * unscale (FP64)
 __global__ __launch_bounds__(kThreads) void k_ref_accum(const RefDev* __restrict__ sys, const int3* __restrict__ work) {
     REF_PROLOGUE
-    const double f = d.unscale[s];
+    const double f = glob(d.unscale)[s];
     if (f == 0.0) return;
     for (int i = g * kThreads + threadIdx.x; i < n; i += stride) {
-        const float2 z = d.d32[base + i];
-        double2 xv = d.x[base + i];
+        const float2 z = glob(d.d32)[base + i];
+        double2 xv = glob(d.x)[base + i];
         xv.x += (double)z.x * f;
         xv.y += (double)z.y * f;
-        d.x[base + i] = xv;
+        glob(d.x)[base + i] = xv;
     }
 }
 
@@ -127,12 +127,12 @@ __global__ __launch_bounds__(kThreads) void k_ref_residual(const RefDev* __restr
     REF_PROLOGUE
     double2 acc[1] = {make_double2(0, 0)};
     for (int i = g * kThreads + threadIdx.x; i < n; i += stride) {
-        const double2 rv = csub(d.b[base + i], d.y[base + i]);
-        d.r[base + i] = rv;
+        const double2 rv = csub(glob(d.b)[base + i], glob(d.y)[base + i]);
+        glob(d.r)[base + i] = rv;
         acc[0].x += rv.x * rv.x + rv.y * rv.y;
     }
     block_sum<1>(acc);
-    if (threadIdx.x == 0) d.part[(size_t)s * d.G + g] = acc[0];
+    if (threadIdx.x == 0) glob(d.part)[(size_t)s * d.G + g] = acc[0];
 }
 
 size_t v64(int n, int S) { return align256(sizeof(double2) * (size_t)n * S); }
@@ -155,8 +155,9 @@ __global__ __launch_bounds__(kThreads) void k_ref_ctl_flat(RefCtl* const* __rest
     const int k = blockIdx.x * kThreads + threadIdx.x;
     if (k >= total) return;
     const int2 c2 = cw[k];
-    if (to_flat) flat[k] = ctlp[c2.x][c2.y];
-    else ctlp[c2.x][c2.y] = flat[k];
+    RefCtl* ctl = glob(ctlp[c2.x]) + c2.y;
+    if (to_flat) flat[k] = *ctl;
+    else *ctl = flat[k];
 }
 
 size_t own_bytes(int n, int S) {
