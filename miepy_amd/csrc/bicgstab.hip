@@ -346,6 +346,7 @@ struct Plan {
     MvDev *d_mv_ps = nullptr, *d_mv_st = nullptr, *d_mv_xt = nullptr;
     int2* d_mv_work[kTileClasses] = {};
     int n_mv_work[kTileClasses] = {};
+    int mv_single[kTileClasses] = {};  // single_job_rows of each list
     Scal* d_scal_out = nullptr;  // gathered scalars, [sum(nrhs)]
     std::vector<char> img;       // host image of the descriptor region, uploaded in one copy
 };
@@ -451,6 +452,7 @@ int build_plan(Plan& P, int nsys, const mpa_system* S_, int dtype, void* scratch
     for (int c = 0; c < kTileClasses; c++) {
         P.d_mv_work[c] = (int2*)p;
         P.n_mv_work[c] = (int)P.mv_work[c].size();
+        P.mv_single[c] = single_job_rows(P.mv_work[c], [&](int i) { return S_[i].n; });
         p += align256(sizeof(int2) * P.mv_work[c].size());
     }
     P.d_scal_out = (Scal*)p;
@@ -491,7 +493,7 @@ int matvec_phase(const Plan& P, const MvDev* d_jobs, const std::vector<MfJob>& m
         if (side) {
             MPA_HIP_CHECK(hipEventRecord(side->fork, st));
             MPA_HIP_CHECK(hipStreamWaitEvent(side->stream, side->fork, 0));
-            const int rc1 = gemv_launch(sizeof(T), d_jobs, P.d_sys, P.d_mv_work, P.n_mv_work, side->stream);
+            const int rc1 = gemv_launch(sizeof(T), d_jobs, P.d_sys, P.d_mv_work, P.n_mv_work, P.mv_single, side->stream);
             const int rc2 = matfree_launch_many(mf, P.d_sys, st);
             // join whatever was launched, also after an error, so no branch is left open
             MPA_HIP_CHECK(hipEventRecord(side->join, side->stream));
@@ -500,7 +502,7 @@ int matvec_phase(const Plan& P, const MvDev* d_jobs, const std::vector<MfJob>& m
         }
     }
     if (any) {
-        const int rc = gemv_launch(sizeof(T), d_jobs, P.d_sys, P.d_mv_work, P.n_mv_work, st);
+        const int rc = gemv_launch(sizeof(T), d_jobs, P.d_sys, P.d_mv_work, P.n_mv_work, P.mv_single, st);
         if (rc) return rc;
     }
     return mf.empty() ? MPA_OK : matfree_launch_many(mf, P.d_sys, st);

@@ -55,21 +55,24 @@ __device__ inline bool all_done(const SysDev& d) {
     return true;
 }
 
-// One workgroup's share of a matvec job: its four waves own R rows each,
-// starting at row 4 R rb; SG right-hand sides per pass, U chunks in flight.
+// One workgroup's share of a matvec job: its four waves own R rows each from
+// row `first` on, up to row `end`; SG right-hand sides per pass, U chunks in
+// flight.  A row's sum is taken in the same order whatever R, SG and U are,
+// so a launch may pick its tile freely.
 template <typename T, int R, int SG, int U>
-__device__ inline void gemv_rows(const MvDev& J, int rb) {
+__device__ inline void gemv_rows(const MvDev& J, int first, int end) {
     using V = typename Chunk<T>::v;
     constexpr int C = Chunk<T>::C;
     const int n = J.n;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int row0 = (rb * 4 + w) * R;
-    if (row0 >= n) return;
+    const int row0 = first + w * R;
+    end = min(end, n);
+    if (row0 >= end) return;
     const int nv = n / C;  // 16-byte chunks per row (n is even)
     const T* A = glob((const T*)J.A);
     const V* Ar[R];
 #pragma unroll
-    for (int r = 0; r < R; r++) Ar[r] = (const V*)(A + (size_t)2 * n * min(row0 + r, n - 1));
+    for (int r = 0; r < R; r++) Ar[r] = (const V*)(A + (size_t)2 * n * min(row0 + r, end - 1));
     for (int s0 = 0; s0 < J.S; s0 += SG) {
         T ar[R][SG], ai[R][SG];
 #pragma unroll
@@ -119,7 +122,7 @@ __device__ inline void gemv_rows(const MvDev& J, int rb) {
                     im += __shfl_xor(im, off);
                 }
                 const int row = row0 + r;
-                if (lane == 0 && row < n && s0 + s < J.S) {
+                if (lane == 0 && row < end && s0 + s < J.S) {
                     const size_t o = (size_t)(s0 + s) * n + row;
                     cplx_t<T> yv = cmake<T>(re, im);
                     if (J.add_identity) yv = cadd(yv, glob((const cplx_t<T>*)J.x)[o]);
@@ -131,465 +134,338 @@ __device__ inline void gemv_rows(const MvDev& J, int rb) {
 
 // ---- multi-RHS products on the matrix cores ------------------------------------
 //
-// Y = (I +) A X for up to kGemmS right-hand sides per pass as a real GEMM:
-// a complex row of A is the real row (Re a_0, Im a_0, Re a_1, ...), and
-// right-hand side s contributes two real columns (one per output part),
+// Y = (I +) A X as a real GEMM: a complex row of A is the real row (Re a_0,
+// Im a_0, Re a_1, ...), and right-hand side s contributes two real columns
+// (one per output part),
 //   X'[2j][(s,re)] = Re x_j,  X'[2j][(s,im)] = Im x_j,
 //   X'[2j+1][(s,re)] = -Im x_j, X'[2j+1][(s,im)] = Re x_j,
 // so that Y_re = sum Re a Re x - Im a Im x and Y_im = sum Re a Im x + Im a Re x.
-// A is streamed once per pass with 16-byte nontemporal loads straight into
-// the MFMA operand registers (each lane reads a contiguous run of its row);
-// the X' block of a K step is staged in LDS once per workgroup and shared by
-// its four waves, whose lanes form their B operands from it.
-//   c64:  v_mfma_f32_32x32x2f32, FP32 accumulate; a wave owns 32 rows x
-//         32 real columns (16 RHS); K step 32 complex columns.
-//   c128: v_mfma_f64_16x16x4f64; a wave owns 16 rows x 2 tiles of 16 real
-//         columns (16 RHS); K step 32 complex columns.
-// Lane layouts (checked on the device): 32x32x2 A lane l -> (row l%32,
-// k l/32), B -> (col l%32, k l/32), D[i] -> (row 8(i/4) + 4(l/32) + i%4,
-// col l%32); f64 16x16x4 A lane l -> (row l%16, k l/16), B -> (col l%16,
-// k l/16), D[i] -> (row 4 i + l/16, col l%16).
+// Eight right-hand sides fill the 16 real columns of one MFMA tile
+// (v_mfma_f32_16x16x4f32 / v_mfma_f64_16x16x4f64).
+//
+// A workgroup owns 16 rows and its W waves split the columns of those rows
+// (wave w takes the K steps w, w + W, ...), so that also a matrix of a few
+// thousand rows gives every CU several independent streams.  A wave moves a K
+// step of its 16 rows and of the right-hand sides from global memory into
+// registers in runs of 64 Q bytes per row, one step ahead, and through its own
+// part of LDS into the MFMA operand layout; nothing is shared between waves,
+// so the loop has no barriers.  At the end the waves' tiles are added in LDS
+// in wave order.  Rows of an LDS buffer are padded by 16 bytes: the 16 rows of
+// one operand read then cover all banks.
+//   A operand: lane l holds row l % 16 and, per 16-byte read, 4 consecutive
+//     reals of c64 (2 complex) or 2 of c128 (1 complex) at the K offset of
+//     its group g = l / 16; its components feed 4 or 2 MFMAs, each with the
+//     X' operand of the same K position (col l % 16: s = col / 2, part = col % 2).
+//   D[i]: row 4 g + i (f32) or 4 i + g (f64), column l % 16.
 
-typedef float f16v __attribute__((ext_vector_type(16)));
 typedef double d4v __attribute__((ext_vector_type(4)));
 
-constexpr int kGemmS = 16;   // right-hand sides per pass
-constexpr int kGemmKB = 32;  // complex columns per K step
-template <typename T> struct GemmRows;
-template <> struct GemmRows<float> { static constexpr int value = 128; };   // 4 waves x 32
-template <> struct GemmRows<double> { static constexpr int value = 64; };   // 4 waves x 16
+constexpr int kGemmS8 = 8;  // right-hand sides per 16-column tile
+constexpr int kGemmW = 8;   // waves per workgroup (the column split)
+constexpr int kGemmQ = 4;   // 64-byte groups of a row per K step
 
-// element of X' for K parity `odd` and output part `part` from x = (re, im)
-template <typename R>
-__device__ inline R xprime(R re, R im, int odd, int part) {
-    return odd ? (part ? re : -im) : (part ? im : re);
+template <typename T> struct MfmaTile;
+template <> struct MfmaTile<float> {
+    using acc = fvec4;
+    static constexpr int C = 2;  // complex entries per 16-byte load
+    __device__ static int row(int g, int i) { return 4 * g + i; }
+    // the 4 K positions of one 16-byte load of A times X'
+    __device__ static void fma(acc& d, fvec4 a, fvec4 x, int part) {
+        d = __builtin_amdgcn_mfma_f32_16x16x4f32(a[0], part ? x.y : x.x, d, 0, 0, 0);
+        d = __builtin_amdgcn_mfma_f32_16x16x4f32(a[1], part ? x.x : -x.y, d, 0, 0, 0);
+        d = __builtin_amdgcn_mfma_f32_16x16x4f32(a[2], part ? x.w : x.z, d, 0, 0, 0);
+        d = __builtin_amdgcn_mfma_f32_16x16x4f32(a[3], part ? x.z : -x.w, d, 0, 0, 0);
+    }
+};
+template <> struct MfmaTile<double> {
+    using acc = d4v;
+    static constexpr int C = 1;
+    __device__ static int row(int g, int i) { return 4 * i + g; }
+    __device__ static void fma(acc& d, dvec2 a, dvec2 x, int part) {
+        d = __builtin_amdgcn_mfma_f64_16x16x4f64(a[0], part ? x.y : x.x, d, 0, 0, 0);
+        d = __builtin_amdgcn_mfma_f64_16x16x4f64(a[1], part ? x.x : -x.y, d, 0, 0, 0);
+    }
+};
+
+// Orders a wave's own LDS writes and reads by different lanes.
+__device__ __forceinline__ void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 }
 
-// A tile of a K step in LDS: rows x (32 complex + 1 pad chunk); the odd
-// 16-byte pad spreads the rows of one MFMA operand read over the banks.
-constexpr int kPadC64 = 2;  // floats of padding per row (c64: 64 + 4 floats -> stride 68 dwords)
+// 16-byte chunks of LDS a wave needs: 16 rows of A and 8 NT of X, 4 Q chunks
+// and one of padding each.
+constexpr int gemm_wave_chunks(int RT, int NT) { return (16 * RT + 8 * NT) * (4 * kGemmQ + 1); }
 
-__device__ inline void gemm_rows_c64(const MvDev& J, int rb) {
-    constexpr int RW = 128, RS = 2 * kGemmKB + 2 * kPadC64;  // rows per workgroup, row stride (floats)
-    __shared__ float As[RW * RS];
-    __shared__ float2 xs[kGemmS][kGemmKB + 1];
+// The right-hand sides [s0, s0 + 8 NT) of rows [r0, r0 + 16 RT).
+template <typename T, int RT, int NT>
+__device__ __forceinline__ void gemm_pass(const MvDev& J, int r0, int s0, typename Chunk<T>::v* lds) {
+    using V = typename Chunk<T>::v;
+    using M = MfmaTile<T>;
+    constexpr int W = kGemmW, Q = kGemmQ, C = M::C, CH = 4 * Q, RS = CH + 1;  // chunks per row and K step; padded row in LDS
+    constexpr int LA = RT * Q, LX = NT * Q / 2;            // loads per lane: 16 (or 8 NT) rows x CH chunks / 64
     const int n = J.n;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int h = lane >> 5, col = lane & 31, s_of = col >> 1, part = col & 1;
-    const float2* A = glob((const float2*)J.A);
-    const float2* X = glob((const float2*)J.x);
-    const int nkb = (n + kGemmKB - 1) / kGemmKB;
-    // global -> register staging of one K step: thread loads 8 chunks of 16 B
-    // (chunk id = it * 256 + tid: 16 chunks per row, a wave covers 4 full rows)
-    for (int s0 = 0; s0 < J.S; s0 += kGemmS) {
-        auto load_a = [&](int kb, fvec4 (&ra)[8]) {
+    const int g = lane >> 4, col = lane & 15, part = col & 1;
+    V* la = lds + w * gemm_wave_chunks(RT, NT);
+    V* lx = la + 16 * RT * RS;
+    // lane's chunk of load k: id = 64 k + lane, row id / CH, chunk id % CH
+    const V* ga[LA];
+    const V* gx[LX];
+    const int ch = lane % CH;
 #pragma unroll
-            for (int it = 0; it < 8; it++) {
-                const int id = it * kThreads + tid;
-                const int r = id >> 4, c16 = id & 15;
-                const int row = min(rb * RW + r, n - 1);
-                const int j = kb * kGemmKB + 2 * c16;  // first complex column of the chunk (even; n even)
-                fvec4 z = {0.f, 0.f, 0.f, 0.f};
-                ra[it] = j < n ? __builtin_nontemporal_load((const fvec4*)(A + (size_t)row * n + j)) : z;
-            }
-        };
-        auto load_x = [&](int kb, float2 (&rx)[2]) {
+    for (int k = 0; k < LA; k++)
+        ga[k] = (const V*)(glob((const cplx_t<T>*)J.A) + (size_t)n * min(r0 + (64 * k + lane) / CH, n - 1));
 #pragma unroll
-            for (int it = 0; it < 2; it++) {
-                const int u = it * kThreads + tid;
-                const int s = u / kGemmKB, jj = u % kGemmKB, j = kb * kGemmKB + jj;
-                rx[it] = (s0 + s < J.S && j < n) ? X[(size_t)(s0 + s) * n + j] : make_float2(0.f, 0.f);
-            }
-        };
-        auto store_lds = [&](const fvec4 (&ra)[8], const float2 (&rx)[2]) {
+    for (int k = 0; k < LX; k++)
+        gx[k] = (const V*)(glob((const cplx_t<T>*)J.x) + (size_t)n * min(s0 + (64 * k + lane) / CH, J.S - 1));
+    typename M::acc acc[RT][NT];
 #pragma unroll
-            for (int it = 0; it < 8; it++) {
-                const int id = it * kThreads + tid;
-                *(fvec4*)(As + (id >> 4) * RS + (id & 15) * 4) = ra[it];
-            }
+    for (int t = 0; t < RT; t++)
 #pragma unroll
-            for (int it = 0; it < 2; it++) {
-                const int u = it * kThreads + tid;
-                xs[u / kGemmKB][u % kGemmKB] = rx[it];
-            }
-        };
-        f16v acc;
+        for (int u = 0; u < NT; u++)
 #pragma unroll
-        for (int i = 0; i < 16; i++) acc[i] = 0.f;
-        fvec4 ra[8];
-        float2 rx[2];
-        load_a(0, ra);
-        load_x(0, rx);
-        for (int kb = 0; kb < nkb; kb++) {
-            __syncthreads();  // the previous step's reads of As / xs are done
-            store_lds(ra, rx);
-            __syncthreads();
-            if (kb + 1 < nkb) {
-                load_a(kb + 1, ra);
-                load_x(kb + 1, rx);
-            }
-            const float* arow = As + (w * 32 + (lane & 31)) * RS + h * 32;
+            for (int i = 0; i < 4; i++) acc[t][u][i] = 0;
+    const int nv = n / C;  // 16-byte chunks per row (n is even)
+    const int steps = (nv + CH - 1) / CH;
+    V a[LA], x[LX];
+    auto load = [&](int kb) {
+        const int c = kb * CH + ch;
+        const bool in = c < nv;
 #pragma unroll
-            for (int q = 0; q < 8; q++) {
-                const fvec4 av = *(const fvec4*)(arow + 4 * q);
+        for (int k = 0; k < LA; k++) a[k] = in ? __builtin_nontemporal_load(ga[k] + c) : V(0);
 #pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const int t = 4 * q + e;
-                    const float2 xv = xs[s_of][16 * h + (t >> 1)];
-                    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av[e], xprime<float>(xv.x, xv.y, t & 1, part), acc, 0, 0,
-                                                               0);
-                }
+        for (int k = 0; k < LX; k++) x[k] = in ? gx[k][c] : V(0);
+    };
+    if (w < steps) load(w);
+    for (int kb = w; kb < steps; kb += W) {
+#pragma unroll
+        for (int k = 0; k < LA; k++) la[(64 * k + lane) / CH * RS + ch] = a[k];
+#pragma unroll
+        for (int k = 0; k < LX; k++) lx[(64 * k + lane) / CH * RS + ch] = x[k];
+        wave_fence();
+        if (kb + W < steps) load(kb + W);
+#pragma unroll
+        for (int q = 0; q < Q; q++) {
+            V av[RT];
+#pragma unroll
+            for (int t = 0; t < RT; t++) av[t] = la[(16 * t + col) * RS + 4 * q + g];
+#pragma unroll
+            for (int u = 0; u < NT; u++) {
+                const V xv = lx[(8 * u + (col >> 1)) * RS + 4 * q + g];
+#pragma unroll
+                for (int t = 0; t < RT; t++) M::fma(acc[t][u], av[t], xv, part);
             }
         }
-        const int s = s0 + s_of;
+        wave_fence();  // the next step's writes stay behind these reads
+    }
+    // the waves' tiles, added in wave order (over the operand buffers)
+    constexpr int TILE = RT * NT * 256;
+    T* red = (T*)lds;
+    __syncthreads();
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const int r = rb * RW + w * 32 + 8 * (i >> 2) + 4 * h + (i & 3);
-            if (r < n && s < J.S && s_of < kGemmS) {
-                const size_t o = 2 * ((size_t)s * n + r) + part;
-                float v = acc[i];
-                if (J.add_identity) v += glob((const float*)J.x)[o];
-                glob((float*)J.y)[o] = v;
-            }
+    for (int t = 0; t < RT; t++)
+#pragma unroll
+        for (int u = 0; u < NT; u++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) red[w * TILE + ((t * NT + u) * 4 + i) * 64 + lane] = acc[t][u][i];
+    __syncthreads();
+    for (int e = tid; e < TILE; e += 64 * W) {
+        T v = red[e];
+#pragma unroll
+        for (int k = 1; k < W; k++) v += red[k * TILE + e];
+        const int l = e & 63, i = (e >> 6) & 3, tu = e >> 8, t = tu / NT, u = tu - t * NT;
+        const int r = r0 + 16 * t + M::row(l >> 4, i), s = s0 + 8 * u + ((l & 15) >> 1);
+        if (r < n && s < J.S) {
+            const size_t o = 2 * ((size_t)s * n + r) + (l & 1);
+            if (J.add_identity) v += glob((const T*)J.x)[o];
+            glob((T*)J.y)[o] = v;
         }
     }
+    __syncthreads();  // before the next pass overwrites the sums
 }
 
-// Eight right-hand sides per pass (16 real columns, one 16x16x4 tile wide):
-// v_mfma_f32_16x16x4f32, a wave owns 32 rows as two 16-row tiles sharing
-// each B operand; half the matrix-core work per byte of A of the 16-RHS
-// form, whose upper 16 columns would be idle at S <= 8.  Each lane reads a
-// float4 of its row (real K 16q + 4g .. +3, g = lane / 16) and feeds its
-// four components to four MFMAs, so MFMA (q, e) covers real K 16q + 4g + e
-// over g; the B operands follow the same order.  D[i] of 16x16x4f32 ->
-// (row 4 (l/16) + i, col l%16).
-constexpr int kGemmS8 = 8;
-
-__device__ inline void gemm_rows_c64_s8(const MvDev& J, int rb) {
-    constexpr int RW = 128, RS = 2 * kGemmKB + 2 * kPadC64;  // rows per workgroup, row stride (floats)
-    __shared__ float As[RW * RS];
-    __shared__ fvec4 xs4[kGemmS8][kGemmKB / 2 + 1];  // two complex per float4; one float4 of padding
-    const int n = J.n;
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int g = lane >> 4, col = lane & 15, s_of = col >> 1, part = col & 1;
-    const float2* A = glob((const float2*)J.A);
-    const float2* X = glob((const float2*)J.x);
-    const int nkb = (n + kGemmKB - 1) / kGemmKB;
-    for (int s0 = 0; s0 < J.S; s0 += kGemmS8) {
-        // A: 128 rows x 16 chunks of 16 B, 8 per thread (a wave covers 4 full rows per it)
-        auto load_a = [&](int kb, fvec4 (&ra)[8]) {
-#pragma unroll
-            for (int it = 0; it < 8; it++) {
-                const int id = it * kThreads + tid;
-                const int r = id >> 4, c16 = id & 15;
-                const int row = min(rb * RW + r, n - 1);
-                const int j = kb * kGemmKB + 2 * c16;
-                fvec4 z = {0.f, 0.f, 0.f, 0.f};
-                ra[it] = j < n ? __builtin_nontemporal_load((const fvec4*)(A + (size_t)row * n + j)) : z;
-            }
-        };
-        // X: 8 right-hand sides x 32 complex, one per thread
-        auto load_x = [&](int kb, float2& rx) {
-            const int s = tid / kGemmKB, jj = tid % kGemmKB, j = kb * kGemmKB + jj;
-            rx = (s0 + s < J.S && j < n) ? X[(size_t)(s0 + s) * n + j] : make_float2(0.f, 0.f);
-        };
-        auto store_lds = [&](const fvec4 (&ra)[8], const float2& rx) {
-#pragma unroll
-            for (int it = 0; it < 8; it++) {
-                const int id = it * kThreads + tid;
-                *(fvec4*)(As + (id >> 4) * RS + (id & 15) * 4) = ra[it];
-            }
-            ((float2*)&xs4[tid / kGemmKB][0])[tid % kGemmKB] = rx;
-        };
-        fvec4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
-        fvec4 ra[8];
-        float2 rx;
-        load_a(0, ra);
-        load_x(0, rx);
-        for (int kb = 0; kb < nkb; kb++) {
-            __syncthreads();  // the previous step's reads of As / xs4 are done
-            store_lds(ra, rx);
-            __syncthreads();
-            if (kb + 1 < nkb) {
-                load_a(kb + 1, ra);
-                load_x(kb + 1, rx);
-            }
-            const float* arow0 = As + (w * 32 + col) * RS + 4 * g;
-            const float* arow1 = arow0 + 16 * RS;
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const fvec4 a0 = *(const fvec4*)(arow0 + 16 * q);
-                const fvec4 a1 = *(const fvec4*)(arow1 + 16 * q);
-                const fvec4 xv = xs4[s_of][4 * q + g];  // complex columns 8q + 2g and 8q + 2g + 1
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const float xr = (e >> 1) ? xv.z : xv.x, xi = (e >> 1) ? xv.w : xv.y;
-                    const float b = xprime<float>(xr, xi, e & 1, part);
-                    acc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a0[e], b, acc0, 0, 0, 0);
-                    acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a1[e], b, acc1, 0, 0, 0);
-                }
-            }
-        }
-        const int s = s0 + s_of;
-#pragma unroll
-        for (int t = 0; t < 2; t++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int r = rb * RW + w * 32 + 16 * t + 4 * g + i;
-                if (r < n && s < J.S) {
-                    const size_t o = 2 * ((size_t)s * n + r) + part;
-                    float v = t ? acc1[i] : acc0[i];
-                    if (J.add_identity) v += glob((const float*)J.x)[o];
-                    glob((float*)J.y)[o] = v;
-                }
-            }
-    }
+// All right-hand sides in passes of 8 NT (A streamed once per pass).
+template <typename T, int RT, int NT>
+__device__ __forceinline__ void gemm_rows(const MvDev& J, int first) {
+    constexpr int ops = kGemmW * gemm_wave_chunks(RT, NT);                         // operand buffers
+    constexpr int sums = kGemmW * RT * NT * 256 * (int)sizeof(T) / 16;             // the waves' tiles
+    __shared__ typename Chunk<T>::v lds[ops > sums ? ops : sums];
+    if (first >= J.n) return;
+    for (int s0 = 0; s0 < J.S; s0 += NT * kGemmS8) gemm_pass<T, RT, NT>(J, first, s0, lds);
 }
 
-constexpr int kPadC128 = 2;  // doubles of padding per row (c128: 64 + 2 doubles -> stride 132 dwords)
+// ---- launches -------------------------------------------------------------------------
+//
+// Work lists name (job, block of `unit` rows), the same list whatever the
+// tile: `sub` workgroups share a block.  A launch whose blocks all belong to
+// one job passes sub = 0: workgroup b then owns the b-th tile of that job.
 
-// NT tiles of 8 right-hand sides per pass (NT = 2: 16 RHS; NT = 1: 8 RHS at
-// half the matrix-core work)
-template <int NT>
-__device__ inline void gemm_rows_c128(const MvDev& J, int rb) {
-    constexpr int RW = 64, RS = 2 * kGemmKB + kPadC128;  // rows per workgroup, row stride (doubles)
-    __shared__ double As[RW * RS];
-    __shared__ double2 xs[kGemmS][kGemmKB + 1];
-    const int n = J.n;
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int g = lane >> 4, col = lane & 15, s_of = col >> 1, part = col & 1;
-    const double2* A = glob((const double2*)J.A);
-    const double2* X = glob((const double2*)J.x);
-    const int nkb = (n + kGemmKB - 1) / kGemmKB;
-    // 64 rows x 32 complex = 2048 chunks of 16 B (one complex each): thread loads 8
-    // (chunk id = it * 256 + tid: 32 chunks per row, a wave covers 2 full rows)
-    for (int s0 = 0; s0 < J.S; s0 += 8 * NT) {
-        auto load_a = [&](int kb, dvec2 (&ra)[8]) {
-#pragma unroll
-            for (int it = 0; it < 8; it++) {
-                const int id = it * kThreads + tid;
-                const int r = id >> 5, c = id & 31;
-                const int row = min(rb * RW + r, n - 1);
-                const int j = kb * kGemmKB + c;
-                dvec2 z = {0.0, 0.0};
-                ra[it] = j < n ? __builtin_nontemporal_load((const dvec2*)(A + (size_t)row * n + j)) : z;
-            }
-        };
-        auto load_x = [&](int kb, double2 (&rx)[2]) {
-#pragma unroll
-            for (int it = 0; it < 2; it++) {
-                const int u = it * kThreads + tid;
-                const int s = u / kGemmKB, jj = u % kGemmKB, j = kb * kGemmKB + jj;
-                rx[it] = (s0 + s < J.S && j < n) ? X[(size_t)(s0 + s) * n + j] : make_double2(0.0, 0.0);
-            }
-        };
-        auto store_lds = [&](const dvec2 (&ra)[8], const double2 (&rx)[2]) {
-#pragma unroll
-            for (int it = 0; it < 8; it++) {
-                const int id = it * kThreads + tid;
-                *(dvec2*)(As + (id >> 5) * RS + (id & 31) * 2) = ra[it];
-            }
-#pragma unroll
-            for (int it = 0; it < 2; it++) {
-                const int u = it * kThreads + tid;
-                xs[u / kGemmKB][u % kGemmKB] = rx[it];
-            }
-        };
-        d4v acc0, acc1;
-#pragma unroll
-        for (int i = 0; i < 4; i++) acc0[i] = acc1[i] = 0.0;
-        dvec2 ra[8];
-        double2 rx[2];
-        load_a(0, ra);
-        load_x(0, rx);
-        for (int kb = 0; kb < nkb; kb++) {
-            __syncthreads();
-            store_lds(ra, rx);
-            __syncthreads();
-            if (kb + 1 < nkb) {
-                load_a(kb + 1, ra);
-                load_x(kb + 1, rx);
-            }
-            const double* arow = As + (w * 16 + (lane & 15)) * RS + g * 16;
-#pragma unroll
-            for (int q = 0; q < 8; q++) {
-                const dvec2 av = *(const dvec2*)(arow + 2 * q);
-#pragma unroll
-                for (int e = 0; e < 2; e++) {
-                    const int t = 2 * q + e;
-                    const double2 x0 = xs[s_of][8 * g + (t >> 1)];
-                    acc0 = __builtin_amdgcn_mfma_f64_16x16x4f64(av[e], xprime<double>(x0.x, x0.y, t & 1, part), acc0, 0,
-                                                                0, 0);
-                    if (NT == 2) {
-                        const double2 x1 = xs[8 + s_of][8 * g + (t >> 1)];
-                        acc1 = __builtin_amdgcn_mfma_f64_16x16x4f64(av[e], xprime<double>(x1.x, x1.y, t & 1, part),
-                                                                    acc1, 0, 0, 0);
-                    }
-                }
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int r = rb * RW + w * 16 + 4 * i + g;
-#pragma unroll
-            for (int c = 0; c < NT; c++) {
-                const int s = s0 + 8 * c + s_of;
-                if (r < n && s < J.S) {
-                    const size_t o = 2 * ((size_t)s * n + r) + part;
-                    double v = c ? acc1[i] : acc0[i];
-                    if (J.add_identity) v += glob((const double*)J.x)[o];
-                    glob((double*)J.y)[o] = v;
-                }
-            }
-        }
-    }
+struct RowRange {
+    int job, first, end;
+};
+__device__ __forceinline__ RowRange rows_of_block(const int2* __restrict__ work, int rows, int unit, int sub) {
+    if (sub == 0) return {work[0].x, (int)blockIdx.x * rows, 0x7fffffff};
+    const int item = blockIdx.x / sub;
+    const int2 wk = work[item];
+    return {wk.x, wk.y * unit + ((int)blockIdx.x - item * sub) * rows, (wk.y + 1) * unit};
 }
 
-// SP right-hand sides per pass: 16 or 8
-template <typename T, int SP>
-__device__ inline void gemm_rows(const MvDev& J, int rb);
-template <>
-__device__ inline void gemm_rows<float, 16>(const MvDev& J, int rb) {
-    gemm_rows_c64(J, rb);
-}
-template <>
-__device__ inline void gemm_rows<float, 8>(const MvDev& J, int rb) {
-    gemm_rows_c64_s8(J, rb);
-}
-template <>
-__device__ inline void gemm_rows<double, 16>(const MvDev& J, int rb) {
-    gemm_rows_c128<2>(J, rb);
-}
-template <>
-__device__ inline void gemm_rows<double, 8>(const MvDev& J, int rb) {
-    gemm_rows_c128<1>(J, rb);
-}
-
-template <typename T, int SP>
-__global__ __launch_bounds__(kThreads) void k_gemm(const MvDev* __restrict__ jobs, const SysDev* __restrict__ sys,
-                                                   const int2* __restrict__ work) {
-    const int2 wk = work[blockIdx.x];
-    const MvDev J = jobs[wk.x];
+template <typename T, int RT, int NT>
+__global__ __launch_bounds__(64 * kGemmW) void k_gemm(const MvDev* __restrict__ jobs, const SysDev* __restrict__ sys,
+                                                      const int2* __restrict__ work, int unit, int sub) {
+    const RowRange q = rows_of_block(work, 16 * RT, unit, sub);
+    const MvDev J = jobs[q.job];
     if (J.skip >= 0 && all_done(sys[J.skip])) return;
-    gemm_rows<T, SP>(J, wk.y);
+    gemm_rows<T, RT, NT>(J, q.first);
 }
 
-template <typename T, int SP>
-__global__ __launch_bounds__(kThreads) void k_gemm1(MvDev J) {
-    gemm_rows<T, SP>(J, blockIdx.x);
+template <typename T, int RT, int NT>
+__global__ __launch_bounds__(64 * kGemmW) void k_gemm1(MvDev J) {
+    gemm_rows<T, RT, NT>(J, blockIdx.x * 16 * RT);
 }
 
-// batched: one workgroup per (job, row block) of the work list
-template <typename T, int RB, int SG, int U>
+template <typename T, int R, int SG, int U>
 __global__ __launch_bounds__(kThreads) void k_gemv(const MvDev* __restrict__ jobs, const SysDev* __restrict__ sys,
-                                                   const int2* __restrict__ work) {
-    const int2 wk = work[blockIdx.x];
-    const MvDev J = jobs[wk.x];
+                                                   const int2* __restrict__ work, int unit, int sub) {
+    const RowRange q = rows_of_block(work, 4 * R, unit, sub);
+    const MvDev J = jobs[q.job];
     if (J.skip >= 0 && all_done(sys[J.skip])) return;
-    gemv_rows<T, RB, SG, U>(J, wk.y);
+    gemv_rows<T, R, SG, U>(J, q.first, q.end);
 }
 
-// one job passed by value: workgroup b owns row block b
-template <typename T, int RB, int SG, int U>
+// one job passed by value
+template <typename T, int R, int SG, int U>
 __global__ __launch_bounds__(kThreads) void k_gemv1(MvDev J) {
-    gemv_rows<T, RB, SG, U>(J, blockIdx.x);
+    gemv_rows<T, R, SG, U>(J, blockIdx.x * 4 * R, J.n);
 }
-
 
 // ---- tile variants ------------------------------------------------------------------
 
+// Variant 0 of a class is chosen per launch by size (auto_variant); the
+// others fix a tile: R rows per wave and U chunks in flight (classes of one
+// and two right-hand sides), or RT 16-row tiles per workgroup of the
+// matrix-core product (SG = 0).
 struct Variant {
-    int R, SG, U;  // vector-ALU tile; R = 0 marks the matrix-core GEMM
+    int R, SG, U;
     const char* name;
 };
-constexpr int kMaxVariants = 5;
+constexpr int kMaxVariants = 9;
 const Variant kVariants[kTileClasses][kMaxVariants] = {
-    {{8, 1, 2, "r8u2"}, {4, 1, 2, "r4u2"}, {8, 1, 4, "r8u4"}, {16, 1, 1, "r16u1"}, {4, 1, 4, "r4u4"}},
-    {{4, 2, 2, "r4u2"}, {2, 2, 2, "r2u2"}, {4, 2, 4, "r4u4"}, {8, 2, 1, "r8u1"}, {0, 0, 0, nullptr}},
-    {{2, 4, 2, "r2u2"}, {1, 4, 2, "r1u2"}, {2, 4, 4, "r2u4"}, {0, 16, 0, "mfma"}, {0, 0, 0, nullptr}},
-    {{0, 16, 0, "mfma"}, {1, 8, 2, "r1s8u2"}, {2, 8, 1, "r2s8u1"}, {0, 8, 0, "mfma8"}, {0, 0, 0, nullptr}},
+    {{0, 1, 0, "auto"}, {8, 1, 2, "r8u2"}, {6, 1, 2, "r6u2"}, {5, 1, 2, "r5u2"}, {4, 1, 2, "r4u2"}, {3, 1, 4, "r3u4"},
+     {2, 1, 4, "r2u4"}, {1, 1, 8, "r1u8"}},
+    {{0, 2, 0, "auto"}, {5, 2, 2, "r5u2"}, {4, 2, 2, "r4u2"}, {3, 2, 2, "r3u2"}, {2, 2, 4, "r2u4"}, {1, 2, 4, "r1u4"}},
+    {{0, 0, 0, "auto"}, {1, 0, 0, "mfma16"}, {2, 0, 0, "mfma32"}},
+    {{0, 0, 0, "auto"}, {1, 0, 0, "mfma16"}, {2, 0, 0, "mfma32"}},
 };
 int g_variant[2][kTileClasses] = {{0, 0, 0, 0}, {0, 0, 0, 0}};  // [es == 8][class]
+
+// rows of a work-list block per class (c64 / c128)
+constexpr int kUnit[2][kTileClasses] = {{32, 16, 128, 128}, {32, 16, 64, 64}};
 
 inline int nvariants(int c) {
     int k = 0;
     while (k < kMaxVariants && kVariants[c][k].name) k++;
     return k;
 }
-inline const Variant& variant_of(int c, int es) { return kVariants[c][g_variant[es == 8][c]]; }
 
-template <typename T>
-int launch_variant(int c, int v, const MvDev* jobs, const SysDev* sys, const int2* work, int nwork, const MvDev* one,
-                   hipStream_t st) {
-    const dim3 grid(nwork), block(kThreads);
-#define MPA_VAR(R_, SG_, U_)                                                                          \
-    do {                                                                                              \
-        if (one) hipLaunchKernelGGL((k_gemv1<T, R_, SG_, U_>), grid, block, 0, st, *one);             \
-        else hipLaunchKernelGGL((k_gemv<T, R_, SG_, U_>), grid, block, 0, st, jobs, sys, work);      \
-    } while (0)
+int rows_of_variant(int c, int v) {
     const Variant& V = kVariants[c][v];
-    if (V.R == 0 && V.SG == 8) {
-        if (one) hipLaunchKernelGGL((k_gemm1<T, 8>), grid, block, 0, st, *one);
-        else hipLaunchKernelGGL((k_gemm<T, 8>), grid, block, 0, st, jobs, sys, work);
-    } else if (V.R == 0) {
-        if (one) hipLaunchKernelGGL((k_gemm1<T, 16>), grid, block, 0, st, *one);
-        else hipLaunchKernelGGL((k_gemm<T, 16>), grid, block, 0, st, jobs, sys, work);
-    } else if (c == 0) {
-        switch (v) {
-            case 0: MPA_VAR(8, 1, 2); break;
-            case 1: MPA_VAR(4, 1, 2); break;
-            case 2: MPA_VAR(8, 1, 4); break;
-            case 3: MPA_VAR(16, 1, 1); break;
-            default: MPA_VAR(4, 1, 4); break;
-        }
-    } else if (c == 1) {
-        switch (v) {
-            case 0: MPA_VAR(4, 2, 2); break;
-            case 1: MPA_VAR(2, 2, 2); break;
-            case 2: MPA_VAR(4, 2, 4); break;
-            default: MPA_VAR(8, 2, 1); break;
-        }
-    } else if (c == 2) {
-        switch (v) {
-            case 0: MPA_VAR(2, 4, 2); break;
-            case 1: MPA_VAR(1, 4, 2); break;
-            default: MPA_VAR(2, 4, 4); break;
-        }
-    } else {
-        switch (v) {
-            case 1: MPA_VAR(1, 8, 2); break;
-            default: MPA_VAR(2, 8, 1); break;
+    return V.SG == 0 ? 16 * V.R : 4 * V.R;
+}
+
+// The tile of a launch over `rows` rows.  A CU streams at its own limit
+// however many workgroups it holds, so a launch takes as long as the CU with
+// the most rows: rounds = ceil(workgroups / 256) times the rows of a
+// workgroup.  The tile with the smallest such count, weighted by what the tile
+// itself costs, is the fastest measured one or within 4 % of it at all of the
+// 27 sizes tried from 592 to 30000 rows.  us per product, this rule and the
+// fixed r8u2 / 128-row tiles that served every size before: n = 592 c128 7.3 and
+// 12.5, 2910 24 and 45, 4500 51 and 69, 9000 189 and 260, 20000 920 and 982; 8
+// right-hand sides c64 5600 46 and 306, 9648 133 and 511, 16000 304 and 844.
+double tile_weight(int c, int R, int es, long rounds) {
+    if (c >= 2) return R == 1 ? 1.05 : 1.0;  // one 16-row tile reads X twice as often as two
+    if (c == 0) {
+        if (R == 8) return rounds <= 2 ? 1.001 : 1.0;  // r4u2 first where both fill the same rounds
+        return R == 1 ? 1.12 : R == 2 ? 1.04 : 1.0;    // x is read R times less often than A
+    }
+    if (R == 5) return es == 8 && rounds == 1 ? 1.5 : 1.0;  // alone on a CU its loads do not cover the latency
+    return R == 1 ? 1.30 : R == 2 ? 1.08 : 1.0;
+}
+
+int auto_variant(int c, long rows, int es) {
+    constexpr long kCus = 256;
+    int best = 1;
+    double best_cost = 1e300;
+    for (int v = 1; v < nvariants(c); v++) {
+        const long tile = rows_of_variant(c, v), rounds = ((rows + tile - 1) / tile + kCus - 1) / kCus;
+        const double cost = (double)(rounds * tile) * tile_weight(c, kVariants[c][v].R, es, rounds);
+        if (cost < best_cost - 1e-9) {
+            best = v;
+            best_cost = cost;
         }
     }
+    return best;
+}
+
+template <typename T, int R, int SG, int U>
+void launch_gemv(const MvDev* jobs, const SysDev* sys, const int2* work, int unit, int sub, unsigned grid,
+                 const MvDev* one, hipStream_t st) {
+    if (one) hipLaunchKernelGGL((k_gemv1<T, R, SG, U>), dim3(grid), dim3(kThreads), 0, st, *one);
+    else hipLaunchKernelGGL((k_gemv<T, R, SG, U>), dim3(grid), dim3(kThreads), 0, st, jobs, sys, work, unit, sub);
+}
+
+template <typename T, int RT, int NT>
+void launch_gemm(const MvDev* jobs, const SysDev* sys, const int2* work, int unit, int sub, unsigned grid,
+                 const MvDev* one, hipStream_t st) {
+    if (one) hipLaunchKernelGGL((k_gemm1<T, RT, NT>), dim3(grid), dim3(64 * kGemmW), 0, st, *one);
+    else hipLaunchKernelGGL((k_gemm<T, RT, NT>), dim3(grid), dim3(64 * kGemmW), 0, st, jobs, sys, work, unit, sub);
+}
+
+// One class of a product: the list `work` (nwork blocks; of one job of n =
+// single_n rows if that is not 0), or the job `one` by value.
+template <typename T>
+int launch_class(int c, const MvDev* jobs, const SysDev* sys, const int2* work, int nwork, int single_n,
+                 const MvDev* one, hipStream_t st) {
+    const int unit = kUnit[sizeof(T) == 8][c];
+    if (one) single_n = one->n;
+    int v = g_variant[sizeof(T) == 8][c];
+    if (v == 0) v = auto_variant(c, single_n ? single_n : (long)nwork * unit, sizeof(T));
+    const Variant& V = kVariants[c][v];
+    const int rows = rows_of_variant(c, v);
+    const int sub = single_n ? 0 : (unit + rows - 1) / rows;
+    const unsigned grid = single_n ? (single_n + rows - 1) / rows : (unsigned)nwork * sub;
+#define MPA_VAR(R_, SG_, U_) \
+    if (V.R == R_ && V.SG == SG_) launch_gemv<T, R_, SG_, U_>(jobs, sys, work, unit, sub, grid, one, st);
+#define MPA_GEMM(RT_, NT_) \
+    if (V.R == RT_ && c == NT_ + 1) launch_gemm<T, RT_, NT_>(jobs, sys, work, unit, sub, grid, one, st);
+    MPA_VAR(8, 1, 2) MPA_VAR(6, 1, 2) MPA_VAR(5, 1, 2) MPA_VAR(4, 1, 2)
+    MPA_VAR(3, 1, 4) MPA_VAR(2, 1, 4) MPA_VAR(1, 1, 8)
+    MPA_VAR(5, 2, 2) MPA_VAR(4, 2, 2) MPA_VAR(3, 2, 2) MPA_VAR(2, 2, 4) MPA_VAR(1, 2, 4)
+    MPA_GEMM(1, 1) MPA_GEMM(2, 1) MPA_GEMM(1, 2) MPA_GEMM(2, 2)
 #undef MPA_VAR
+#undef MPA_GEMM
     MPA_LAUNCH_CHECK();
     return MPA_OK;
 }
 
-int rows_of_variant(int c, int v, int es) {
-    const Variant& V = kVariants[c][v];
-    if (V.R == 0) return es == 8 ? GemmRows<double>::value : GemmRows<float>::value;
-    return 4 * V.R;
-}
-
 }  // namespace
 
-int gemv_class(int S) { return S == 1 ? 0 : (S == 2 ? 1 : (S <= 4 ? 2 : 3)); }
-
-int gemv_rows_of_class(int c, int es) { return rows_of_variant(c, g_variant[es == 8][c], es); }
+int gemv_class(int S) { return S == 1 ? 0 : (S == 2 ? 1 : (S <= 8 ? 2 : 3)); }
 
 int gemv_row_blocks(int n, int S, int es) {
-    const int rb = gemv_rows_of_class(gemv_class(S), es);
-    return (n + rb - 1) / rb;
+    const int unit = kUnit[es == 8][gemv_class(S)];
+    return (n + unit - 1) / unit;
 }
 
-int gemv_launch(int es, const MvDev* jobs, const SysDev* sys, int2* const* work, const int* nwork, hipStream_t st) {
+int gemv_launch(int es, const MvDev* jobs, const SysDev* sys, int2* const* work, const int* nwork,
+                const int* single_n, hipStream_t st) {
     ProfScope prof(es == 8 ? 0 : 1, st);
     for (int c = 0; c < kTileClasses; c++) {
         if (!nwork[c]) continue;
-        const int v = g_variant[es == 8][c];
-        const int rc = es == 8 ? launch_variant<double>(c, v, jobs, sys, work[c], nwork[c], nullptr, st)
-                               : launch_variant<float>(c, v, jobs, sys, work[c], nwork[c], nullptr, st);
+        const int rc = es == 8
+                           ? launch_class<double>(c, jobs, sys, work[c], nwork[c], single_n[c], nullptr, st)
+                           : launch_class<float>(c, jobs, sys, work[c], nwork[c], single_n[c], nullptr, st);
         if (rc) return rc;
     }
     return MPA_OK;
@@ -598,10 +474,8 @@ int gemv_launch(int es, const MvDev* jobs, const SysDev* sys, int2* const* work,
 int gemv_launch1(int es, const MvDev& J, hipStream_t st) {
     ProfScope prof(es == 8 ? 0 : 1, st);
     const int c = gemv_class(J.S);
-    const int v = g_variant[es == 8][c];
-    const int nb = (J.n + rows_of_variant(c, v, es) - 1) / rows_of_variant(c, v, es);
-    return es == 8 ? launch_variant<double>(c, v, nullptr, nullptr, nullptr, nb, &J, st)
-                   : launch_variant<float>(c, v, nullptr, nullptr, nullptr, nb, &J, st);
+    return es == 8 ? launch_class<double>(c, nullptr, nullptr, nullptr, 0, 0, &J, st)
+                   : launch_class<float>(c, nullptr, nullptr, nullptr, 0, 0, &J, st);
 }
 
 }  // namespace mpa
@@ -686,17 +560,15 @@ extern "C" int mpa_autotune_matvec_batched(int count, const int* n, const int* n
         if (gemv_class(nrhs[i]) == c) jobs.push_back(MvDev{A[i], x[i], y[i], n[i], nrhs[i], 0, -1});
     }
     const int nv = nvariants(c);
-    size_t max_work = 0;
-    for (int v = 0; v < nv; v++) {
-        size_t w = 0;
-        for (const MvDev& J : jobs) w += (J.n + rows_of_variant(c, v, es) - 1) / rows_of_variant(c, v, es);
-        max_work = w > max_work ? w : max_work;
-    }
+    std::vector<int2> work;
+    for (int j = 0; j < (int)jobs.size(); j++)
+        for (int b = 0; b < gemv_row_blocks(jobs[j].n, jobs[j].S, es); b++) work.push_back(make_int2(j, b));
+    order_work_longest_first(work, [&](int j) { return jobs[j].n; });  // as the solvers order it
     hipStream_t st = (hipStream_t)stream;
     MvDev* d_jobs = nullptr;
     int2* d_work = nullptr;
     MPA_HIP_CHECK(hipMalloc(&d_jobs, sizeof(MvDev) * jobs.size()));
-    if (hipMalloc(&d_work, sizeof(int2) * max_work) != hipSuccess) {
+    if (hipMalloc(&d_work, sizeof(int2) * work.size()) != hipSuccess) {
         (void)hipFree(d_jobs);
         mpa_set_error("autotune_matvec_batched: out of device memory");
         return MPA_ERR_OOM;
@@ -704,32 +576,23 @@ extern "C" int mpa_autotune_matvec_batched(int count, const int* n, const int* n
     hipEvent_t e0 = nullptr, e1 = nullptr;
     int rc = MPA_OK;
     if (hipMemcpyAsync(d_jobs, jobs.data(), sizeof(MvDev) * jobs.size(), hipMemcpyHostToDevice, st) != hipSuccess ||
+        hipMemcpyAsync(d_work, work.data(), sizeof(int2) * work.size(), hipMemcpyHostToDevice, st) != hipSuccess ||
         hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess)
         rc = MPA_ERR_HIP;
     const int saved = g_variant[es == 8][c];
     int best = saved;
     double best_ms = 1e30;
-    std::vector<int2> work;
     for (int v = 0; v < nv && rc == MPA_OK; v++) {
-        const int rows = rows_of_variant(c, v, es);
-        work.clear();
-        for (int j = 0; j < (int)jobs.size(); j++)
-            for (int b = 0; b < (jobs[j].n + rows - 1) / rows; b++) work.push_back(make_int2(j, b));
-        order_work_longest_first(work, [&](int j) { return jobs[j].n; });  // as the solvers order it
-        if (hipMemcpyAsync(d_work, work.data(), sizeof(int2) * work.size(), hipMemcpyHostToDevice, st) != hipSuccess ||
-            hipStreamSynchronize(st) != hipSuccess) {
-            rc = MPA_ERR_HIP;
-            break;
-        }
         g_variant[es == 8][c] = v;
         int2* wl[kTileClasses] = {nullptr, nullptr, nullptr, nullptr};
-        int nw[kTileClasses] = {0, 0, 0, 0};
+        int nw[kTileClasses] = {0, 0, 0, 0}, single[kTileClasses] = {0, 0, 0, 0};
         wl[c] = d_work;
         nw[c] = (int)work.size();
-        rc = gemv_launch(es, d_jobs, nullptr, wl, nw, st);  // warm-up
+        single[c] = jobs.size() == 1 ? jobs[0].n : 0;
+        rc = gemv_launch(es, d_jobs, nullptr, wl, nw, single, st);  // warm-up
         if (rc) break;
         (void)hipEventRecord(e0, st);
-        for (int r = 0; r < reps && rc == MPA_OK; r++) rc = gemv_launch(es, d_jobs, nullptr, wl, nw, st);
+        for (int r = 0; r < reps && rc == MPA_OK; r++) rc = gemv_launch(es, d_jobs, nullptr, wl, nw, single, st);
         (void)hipEventRecord(e1, st);
         if (hipEventSynchronize(e1) != hipSuccess) rc = MPA_ERR_HIP;
         float ms = 0;

@@ -189,8 +189,8 @@ bool valid(int nsys, const mpa_refine_system* s) {
 // both present (and MPA_OPT_OVERLAP) the GEMV runs on the device's side
 // stream beside the matrix-free products, joined before the caller's next
 // launch, as in the solver's product phases.
-int residual_products(const MvDev* d_mv, int2* const* d_mw, const int* n_mw, const std::vector<MfJob>& mf,
-                      hipStream_t st) {
+int residual_products(const MvDev* d_mv, int2* const* d_mw, const int* n_mw, const int* single_n,
+                      const std::vector<MfJob>& mf, hipStream_t st) {
     bool any_mv = false;
     for (int c = 0; c < kTileClasses; c++) any_mv |= n_mw[c] > 0;
     if (any_mv && !mf.empty() && mpa_option(MPA_OPT_OVERLAP) != 0 && !mpa_profile_active()) {
@@ -199,7 +199,7 @@ int residual_products(const MvDev* d_mv, int2* const* d_mw, const int* n_mw, con
         if (side) {
             MPA_HIP_CHECK(hipEventRecord(side->fork, st));
             MPA_HIP_CHECK(hipStreamWaitEvent(side->stream, side->fork, 0));
-            const int rc1 = gemv_launch(8, d_mv, nullptr, d_mw, n_mw, side->stream);
+            const int rc1 = gemv_launch(8, d_mv, nullptr, d_mw, n_mw, single_n, side->stream);
             const int rc2 = matfree_launch_many(mf, nullptr, st);
             MPA_HIP_CHECK(hipEventRecord(side->join, side->stream));
             MPA_HIP_CHECK(hipStreamWaitEvent(st, side->join, 0));
@@ -207,7 +207,7 @@ int residual_products(const MvDev* d_mv, int2* const* d_mw, const int* n_mw, con
         }
     }
     int rc = MPA_OK;
-    if (any_mv && (rc = gemv_launch(8, d_mv, nullptr, d_mw, n_mw, st))) return rc;
+    if (any_mv && (rc = gemv_launch(8, d_mv, nullptr, d_mw, n_mw, single_n, st))) return rc;
     if (!mf.empty() && (rc = matfree_launch_many(mf, nullptr, st))) return rc;
     return MPA_OK;
 }
@@ -276,10 +276,11 @@ int refine_batch(int nsys, const mpa_refine_system* R, void* scratch, int* outer
     int3* d_vw = (int3*)p; p += align256(sizeof(int3) * vw.size());
     int2* d_cw = (int2*)p; p += align256(sizeof(int2) * cw.size());
     int2* d_mw[kTileClasses];
-    int n_mw[kTileClasses];
+    int n_mw[kTileClasses], single_n[kTileClasses];
     for (int c = 0; c < kTileClasses; c++) {
         d_mw[c] = (int2*)p;
         n_mw[c] = (int)mw[c].size();
+        single_n[c] = single_job_rows(mw[c], [&](int i) { return R[i].n; });
         p += align256(sizeof(int2) * mw[c].size());
     }
     double* d_flat = (double*)p;  // [3 total]: gathered norms, scale, unscale
@@ -379,7 +380,7 @@ int refine_batch(int nsys, const mpa_refine_system* R, void* scratch, int* outer
             }
         hipLaunchKernelGGL(k_ref_accum, dim3(nv), dim3(kThreads), 0, st, d_ref, d_vw);
         MPA_LAUNCH_CHECK();
-        if ((rc = residual_products(d_mv, d_mw, n_mw, mf, st))) return rc;
+        if ((rc = residual_products(d_mv, d_mw, n_mw, single_n, mf, st))) return rc;
         hipLaunchKernelGGL(k_ref_residual, dim3(nv), dim3(kThreads), 0, st, d_ref, d_vw);
         hipLaunchKernelGGL(k_ref_norms, dim3(nc), dim3(kThreads), 0, st, d_ref, d_cw);
         MPA_LAUNCH_CHECK();
@@ -547,7 +548,7 @@ int refine_iterate(int nsys, const mpa_refine_system* R, void* scratch, bool sta
     // pageable source: staged by the runtime before the call returns
     MPA_HIP_CHECK(hipMemcpyAsync(ctl_region, ctl_img.data(), ctl_head, hipMemcpyHostToDevice, st));
     const unsigned ctl_grid = (unsigned)((total + kThreads - 1) / kThreads);
-    auto upload = [&](const SubLists& L, int2** d_mw, int* n_mw) -> int {
+    auto upload = [&](const SubLists& L, int2** d_mw, int* n_mw, int* single_n) -> int {
         if (!L.vw.empty())
             MPA_HIP_CHECK(hipMemcpyAsync(d_vw, L.vw.data(), sizeof(int3) * L.vw.size(), hipMemcpyHostToDevice, st));
         if (!L.cw.empty())
@@ -556,6 +557,7 @@ int refine_iterate(int nsys, const mpa_refine_system* R, void* scratch, bool sta
         for (int c = 0; c < kTileClasses; c++) {
             d_mw[c] = (int2*)q;
             n_mw[c] = (int)L.mw[c].size();
+            single_n[c] = single_job_rows(L.mw[c], [&](int i) { return R[i].n; });
             if (n_mw[c])
                 MPA_HIP_CHECK(hipMemcpyAsync(d_mw[c], L.mw[c].data(), sizeof(int2) * n_mw[c], hipMemcpyHostToDevice, st));
             q += align256(sizeof(int2) * L.mw[c].size());
@@ -563,7 +565,7 @@ int refine_iterate(int nsys, const mpa_refine_system* R, void* scratch, bool sta
         return MPA_OK;
     };
     int2* d_mw[kTileClasses];
-    int n_mw[kTileClasses];
+    int n_mw[kTileClasses], single_n[kTileClasses];
     std::vector<RefCtl> ctl(total);
     std::vector<double> nrm(total);
     auto read_ctl = [&]() -> int {
@@ -610,7 +612,7 @@ int refine_iterate(int nsys, const mpa_refine_system* R, void* scratch, bool sta
     if (start) {
         // x = 0, r = b, ||b||^2; every system starts in the decision phase
         SubLists L = sub_lists(all, R, V);
-        if ((rc = upload(L, d_mw, n_mw))) return rc;
+        if ((rc = upload(L, d_mw, n_mw, single_n))) return rc;
         hipLaunchKernelGGL(k_ref_start, dim3((unsigned)L.vw.size()), dim3(kThreads), 0, st, d_ref, d_vw);
         hipLaunchKernelGGL(k_ref_norms, dim3((unsigned)L.cw.size()), dim3(kThreads), 0, st, d_ref, d_cw);
         MPA_LAUNCH_CHECK();
@@ -656,10 +658,10 @@ int refine_iterate(int nsys, const mpa_refine_system* R, void* scratch, bool sta
     // B. finished corrections: x += ||r|| d, FP64 residual and norms
     if (!finished_inner.empty()) {
         SubLists L = sub_lists(finished_inner, R, V);
-        if ((rc = upload(L, d_mw, n_mw))) return rc;
+        if ((rc = upload(L, d_mw, n_mw, single_n))) return rc;
         hipLaunchKernelGGL(k_ref_accum, dim3((unsigned)L.vw.size()), dim3(kThreads), 0, st, d_ref, d_vw);
         MPA_LAUNCH_CHECK();
-        if ((rc = residual_products(d_mv, d_mw, n_mw, L.mf, st))) return rc;
+        if ((rc = residual_products(d_mv, d_mw, n_mw, single_n, L.mf, st))) return rc;
         hipLaunchKernelGGL(k_ref_residual, dim3((unsigned)L.vw.size()), dim3(kThreads), 0, st, d_ref, d_vw);
         hipLaunchKernelGGL(k_ref_norms, dim3((unsigned)L.cw.size()), dim3(kThreads), 0, st, d_ref, d_cw);
         MPA_LAUNCH_CHECK();
@@ -691,7 +693,7 @@ int refine_iterate(int nsys, const mpa_refine_system* R, void* scratch, bool sta
             // them is decided afresh below, which sets its scales again before any further use)
             if ((rc = write_scales(flat_host, cnt, 2))) return rc;
             SubLists Lr = sub_lists(revert_sys, R, V);
-            if ((rc = upload(Lr, d_mw, n_mw))) return rc;
+            if ((rc = upload(Lr, d_mw, n_mw, single_n))) return rc;
             hipLaunchKernelGGL(k_ref_accum, dim3((unsigned)Lr.vw.size()), dim3(kThreads), 0, st, d_ref, d_vw);
             MPA_LAUNCH_CHECK();
         }
@@ -734,7 +736,7 @@ int refine_iterate(int nsys, const mpa_refine_system* R, void* scratch, bool sta
         }
         if (!starting.empty()) {
             SubLists L = sub_lists(starting, R, V);
-            if ((rc = upload(L, d_mw, n_mw))) return rc;
+            if ((rc = upload(L, d_mw, n_mw, single_n))) return rc;
             // scale = 1 / ||r||, unscale = ||r|| of every RHS that starts a correction (0 for the others),
             // in the order of the starting set's (system, RHS) list
             const int cnt = (int)L.cw.size();
