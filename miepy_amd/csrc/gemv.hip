@@ -198,7 +198,7 @@ __device__ __forceinline__ void wave_fence() {
 constexpr int gemm_wave_chunks(int RT, int NT) { return (16 * RT + 8 * NT) * (4 * kGemmQ + 1); }
 
 // The right-hand sides [s0, s0 + 8 NT) of rows [r0, r0 + 16 RT).
-template <typename T, int RT, int NT>
+template <typename T, int RT, int NT, bool STREAM>
 __device__ __forceinline__ void gemm_pass(const MvDev& J, int r0, int s0, typename Chunk<T>::v* lds) {
     using V = typename Chunk<T>::v;
     using M = MfmaTile<T>;
@@ -232,8 +232,13 @@ __device__ __forceinline__ void gemm_pass(const MvDev& J, int r0, int s0, typena
     auto load = [&](int kb) {
         const int c = kb * CH + ch;
         const bool in = c < nv;
+        if (STREAM) {
 #pragma unroll
-        for (int k = 0; k < LA; k++) a[k] = in ? __builtin_nontemporal_load(ga[k] + c) : V(0);
+            for (int k = 0; k < LA; k++) a[k] = in ? __builtin_nontemporal_load(ga[k] + c) : V(0);
+        } else {
+#pragma unroll
+            for (int k = 0; k < LA; k++) a[k] = in ? ga[k][c] : V(0);
+        }
 #pragma unroll
         for (int k = 0; k < LX; k++) x[k] = in ? gx[k][c] : V(0);
     };
@@ -292,7 +297,13 @@ __device__ __forceinline__ void gemm_rows(const MvDev& J, int first) {
     constexpr int sums = kGemmW * RT * NT * 256 * (int)sizeof(T) / 16;             // the waves' tiles
     __shared__ typename Chunk<T>::v lds[ops > sums ? ops : sums];
     if (first >= J.n) return;
-    for (int s0 = 0; s0 < J.S; s0 += NT * kGemmS8) gemm_pass<T, RT, NT>(J, first, s0, lds);
+    // Rows of whole 128-byte lines are streamed past the caches (c64, 8 sources, n = 9648: 133 us, 142 through
+    // them).  Otherwise neighbouring steps share lines, which the caches then serve (n = 9990: 174 us, 183).
+    if (J.n % (128 / (2 * (int)sizeof(T))) == 0) {
+        for (int s0 = 0; s0 < J.S; s0 += NT * kGemmS8) gemm_pass<T, RT, NT, true>(J, first, s0, lds);
+    } else {
+        for (int s0 = 0; s0 < J.S; s0 += NT * kGemmS8) gemm_pass<T, RT, NT, false>(J, first, s0, lds);
+    }
 }
 
 // ---- launches -------------------------------------------------------------------------
