@@ -143,3 +143,34 @@ def test_lu_large_system(dev):
     dt = time.perf_counter() - t0
     print(f"LU solve n={n}: {dt * 1e3:.1f} ms")
     assert np.linalg.norm(A @ x[0] - b[0]) <= 1e-13 * np.linalg.norm(A) * np.linalg.norm(x[0])
+
+
+@pytest.mark.parametrize("n,S", [(513, 1), (608, 5), (1100, 3), (2081, 1), (3076, 1), (3300, 2)])
+def test_lu_strips(dev, n, S):
+    """Row counts on both sides of each strip of the panel factorization (512,
+    1024, 2048 and 3072 rows in a workgroup's registers, 8 and 4 columns), a
+    Gaussian matrix (a pivot from below in nearly every column): the residual
+    bar of the oracle tests, |L| <= 1 and L U = P A on a sample of rows."""
+    import torch
+    g = torch.Generator().manual_seed(n)
+    A = torch.randn((n, n), dtype=torch.complex128, generator=g)
+    b = torch.randn((S, n), dtype=torch.complex128, generator=g)
+    F = A.to("cuda")
+    x = dev.lu_solve(F, b.to("cuda"), overwrite=True).cpu()
+    for s in range(S):
+        assert (A @ x[s] - b[s]).norm() <= 1e-13 * A.norm() * x[s].norm()
+    LU = F.cpu()
+    L = torch.tril(LU, -1)
+    assert L.abs().max() <= 1 + 1e-12
+    rows = torch.linspace(0, n - 1, 7).long()
+    PA = (L[rows] + torch.eye(n, dtype=LU.dtype)[rows]) @ torch.triu(LU)
+    for r in PA:  # every row of L U is a row of A
+        assert (A - r).abs().max(dim=1).values.min() <= 1e-12 * A.abs().max() * n ** 0.5
+
+
+def test_lu_singular_column_inside_a_strip(dev):
+    rng = np.random.default_rng(12)
+    A, b = _random(rng, 640, 1)
+    A[:, 531] = 0.0
+    with pytest.raises(np.linalg.LinAlgError, match="column 531"):
+        dev.lu_solve(dev.to_device(A, dev.C128), dev.to_device(b, dev.C128))
