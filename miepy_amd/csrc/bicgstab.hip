@@ -94,6 +94,7 @@ __global__ __launch_bounds__(kThreads) void k_init_scalars(const SysDev* __restr
         c.status = MPA_OK;
         c.restart_pending = 0;
         c.init_pending = 0;
+        c.p_ready = 0;
         c.rho_next = make_double2(bb.x, 0);  // <r0, r> = ||b||^2 with x0 = 0
         if (ref) {
             // x0 = b: the restart kernels form r = b - A b, r0 = r and make the
@@ -117,7 +118,7 @@ __global__ __launch_bounds__(kThreads) void k_update_p(const SysDev* __restrict_
     using C = cplx_t<T>;
     VEC_PROLOGUE
     const Scal& c = glob(d.scal)[s];
-    if (c.done || c.restart_pending) return;
+    if (c.done || c.restart_pending || c.p_ready) return;
     const double2 beta = cmul(cdiv(c.rho_next, c.rho), cdiv(c.alpha, c.w));
     const C bt = from_d<T>(beta), wt = from_d<T>(c.w);
     C *p = glob((C*)d.p), *r = glob((C*)d.r), *v = glob((C*)d.v);
@@ -177,7 +178,10 @@ __global__ __launch_bounds__(kThreads) void k_update_s(const SysDev* __restrict_
     const C at = from_d<T>(alpha);
     C *sv = glob((C*)d.s), *r = glob((C*)d.r), *v = glob((C*)d.v);
     for (int i = g * kThreads + threadIdx.x; i < n; i += stride) sv[base + i] = csub(r[base + i], cmul(at, v[base + i]));
-    if (g == 0 && threadIdx.x == 0) glob(d.scal)[s].alpha_next = alpha;
+    if (g == 0 && threadIdx.x == 0) {
+        glob(d.scal)[s].alpha_next = alpha;
+        glob(d.scal)[s].p_ready = 0;
+    }
 }
 
 // partials <t, s>, <t, t>
@@ -232,7 +236,29 @@ __global__ __launch_bounds__(kThreads) void k_update_xr(const SysDev* __restrict
     if (g == 0 && threadIdx.x == 0) glob(d.scal)[s].w_next = om;
 }
 
-// commit the iteration's scalars; convergence, maxiter and restart checks
+// An iteration's scalars from ||r||^2 and <r0, r>; convergence, maxiter and restart checks.
+__device__ __forceinline__ void commit_scalars(Scal& c, double rr, double2 r0r, bool ref) {
+    c.rho = c.rho_next;
+    c.alpha = c.alpha_next;
+    c.w = c.w_next;
+    c.rnorm2 = rr;
+    c.it += 1;
+    c.rho_next = r0r;
+    const double eps = 2.220446049250313e-16;  // NumTraits<double>::epsilon()
+    if (!(rr == rr) || !(r0r.x == r0r.x) || !(r0r.y == r0r.y)) {
+        c.done = 1;
+        c.status = MPA_NONFINITE;
+    } else if (ref ? rr < c.tol2 : !(rr > c.tol2)) {  // ||r|| < tol (reference loop), Eigen's <=
+        c.done = 1;
+    } else if (c.it >= c.maxiter) {
+        c.done = 1;
+        c.status = MPA_NOT_CONVERGED;
+    } else if (!ref && sqrt(r0r.x * r0r.x + r0r.y * r0r.y) < eps * eps * c.r0_sq) {
+        c.restart_pending = 1;
+    }
+}
+
+// commit the iteration's scalars
 __global__ __launch_bounds__(kThreads) void k_commit(const SysDev* __restrict__ sys, const int2* __restrict__ cw) {
     const int2 c2 = cw[blockIdx.x];
     const SysDev& d = sys[c2.x];
@@ -242,25 +268,154 @@ __global__ __launch_bounds__(kThreads) void k_commit(const SysDev* __restrict__ 
     const double2 rr = reduce_partials(d.part, d.G, s, 3);
     const double2 r0r = reduce_partials(d.part, d.G, s, 4);
     if (threadIdx.x == 0) {
-        c.rho = c.rho_next;
-        c.alpha = c.alpha_next;
-        c.w = c.w_next;
-        c.rnorm2 = rr.x;
-        c.it += 1;
-        c.rho_next = r0r;
-        const double eps = 2.220446049250313e-16;  // NumTraits<double>::epsilon()
-        const bool ref = (d.flags & MPA_SOLVE_REF_LOOP) != 0;
-        if (!(rr.x == rr.x) || !(r0r.x == r0r.x) || !(r0r.y == r0r.y)) {
-            c.done = 1;
-            c.status = MPA_NONFINITE;
-        } else if (ref ? rr.x < c.tol2 : !(rr.x > c.tol2)) {  // ||r|| < tol (reference loop), Eigen's <=
-            c.done = 1;
-        } else if (c.it >= c.maxiter) {
-            c.done = 1;
-            c.status = MPA_NOT_CONVERGED;
-        } else if (!ref && sqrt(r0r.x * r0r.x + r0r.y * r0r.y) < eps * eps * c.r0_sq) {
-            c.restart_pending = 1;
+        Scal next = c;
+        commit_scalars(next, rr.x, r0r, (d.flags & MPA_SOLVE_REF_LOOP) != 0);
+        c = next;
+    }
+}
+
+// ---- the vector work of a half iteration in one workgroup per (system, RHS) ------
+//
+// Up to kHalfMaxN unknowns one workgroup per right-hand side does what the
+// kernels above do in two and four launches, whose fixed 4-5 us each were most
+// of a small solve's time: k_half1 <r0, v>, alpha and s; k_half2 <t, s>, <t, t>,
+// w, x, r, ||r||^2, <r0, r>, the commit and the next direction p.  The sums are
+// taken in the same order as there: element i = g 256 + t + k G 256 belongs to
+// thread t of group g, a group is summed by wave and then over its 4 waves, the
+// G group sums as reduce_partials does.  So a system's iterates do not depend
+// on which kernels its batch uses.  us per iteration, products included, one
+// source: n = 592 40.8 -> 34.7, n = 1800 55.2 -> 46.7; at n = 4500 one CU's
+// bandwidth takes the gain back (133.7 and 134.6, two passes).
+constexpr int kHalfT = 1024;      // threads: 4 groups of 256
+constexpr int kHalfMaxN = 4096;   // 4 groups of 1024 elements
+
+// Sums of K values over the group sums of all G groups; the result is in every thread.
+template <int K>
+__device__ __forceinline__ void half_sum(const double2 (&v)[K], int G, double2 (&out)[K],
+                                         double2 (*red)[kHalfT / 64]) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+        double re = v[k].x, im = v[k].y;
+        for (int off = 32; off > 0; off >>= 1) {
+            re += __shfl_xor(re, off);
+            im += __shfl_xor(im, off);
         }
+        if (lane == 0) red[k][wave] = make_double2(re, im);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+        double2 s = make_double2(0, 0);
+        if (lane < G) {  // group `lane`: waves 4 lane ..
+            const double2* w = red[k] + 4 * lane;
+            s = w[0];
+            for (int q = 1; q < 4; q++) s = cadd(s, w[q]);
+        }
+        double re = s.x, im = s.y;
+        for (int off = 32; off > 0; off >>= 1) {
+            re += __shfl_xor(re, off);
+            im += __shfl_xor(im, off);
+        }
+        out[k] = make_double2(re, im);
+    }
+}
+
+#define HALF_PROLOGUE                                                                            \
+    using C = cplx_t<T>;                                                                         \
+    const int2 c2 = cw[blockIdx.x];                                                              \
+    const SysDev& d = sys[c2.x];                                                                 \
+    const int s = c2.y, n = d.n, G = d.G;                                                        \
+    const size_t base = (size_t)s * n;                                                           \
+    Scal* sc = glob(d.scal) + s;                                                                 \
+    if (sc->done || sc->restart_pending) return;                                                 \
+    __shared__ double2 red[2][2][kHalfT / 64];                                                   \
+    /* the k-th element of this thread in its group threadIdx.x / 256 */                         \
+    auto index = [&](int k) {                                                                    \
+        const int i = (int)threadIdx.x + k * G * kThreads;                                       \
+        return (int)(threadIdx.x >> 8) < G && i < n ? i : -1;                                    \
+    };
+
+template <typename T>
+__global__ __launch_bounds__(kHalfT) void k_half1(const SysDev* __restrict__ sys, const int2* __restrict__ cw) {
+    HALF_PROLOGUE
+    const C *r0 = glob((const C*)d.r0) + base, *v = glob((const C*)d.v) + base, *r = glob((const C*)d.r) + base;
+    C* sv = glob((C*)d.s) + base;
+    C vv[4], rv[4];
+    double2 acc[1] = {make_double2(0, 0)}, dv[1];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const int i = index(e);
+        if (i < 0) continue;
+        vv[e] = v[i];
+        rv[e] = r[i];
+        acc[0] = cadd(acc[0], cmulc(to_d(r0[i]), to_d(vv[e])));
+    }
+    half_sum<1>(acc, G, dv, red[0]);
+    const double2 alpha = cdiv(sc->rho_next, dv[0]);
+    const C at = from_d<T>(alpha);
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const int i = index(e);
+        if (i >= 0) sv[i] = csub(rv[e], cmul(at, vv[e]));
+    }
+    if (threadIdx.x == 0) {
+        sc->alpha_next = alpha;
+        sc->p_ready = 0;
+    }
+}
+
+template <typename T>
+__global__ __launch_bounds__(kHalfT) void k_half2(const SysDev* __restrict__ sys, const int2* __restrict__ cw) {
+    HALF_PROLOGUE
+    const C *r0 = glob((const C*)d.r0) + base, *v = glob((const C*)d.v) + base, *sv = glob((const C*)d.s) + base;
+    const C* tv = glob((const C*)d.t) + base;
+    C *x = glob((C*)d.x) + base, *p = glob((C*)d.p) + base, *r = glob((C*)d.r) + base;
+    Scal next = *sc;
+    C st[4], tt[4];
+    double2 acc[2] = {make_double2(0, 0), make_double2(0, 0)}, sum[2];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const int i = index(e);
+        if (i < 0) continue;
+        st[e] = sv[i];
+        tt[e] = tv[i];
+        const double2 t = to_d(tt[e]);
+        acc[0] = cadd(acc[0], cmulc(t, to_d(st[e])));
+        acc[1].x += t.x * t.x + t.y * t.y;
+    }
+    half_sum<2>(acc, G, sum, red[0]);
+    const double2 om = sum[1].x > 0 ? cscale(sum[0], 1.0 / sum[1].x) : make_double2(0, 0);
+    const C at = from_d<T>(next.alpha_next), wt = from_d<T>(om);
+    acc[0] = acc[1] = make_double2(0, 0);
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const int i = index(e);
+        if (i < 0) continue;
+        x[i] = cadd(x[i], cadd(cmul(at, p[i]), cmul(wt, st[e])));
+        const C rv = csub(st[e], cmul(wt, tt[e]));
+        r[i] = rv;
+        st[e] = rv;
+        const double2 rd = to_d(rv);
+        acc[0].x += rd.x * rd.x + rd.y * rd.y;
+        acc[1] = cadd(acc[1], cmulc(to_d(r0[i]), rd));
+    }
+    half_sum<2>(acc, G, sum, red[1]);
+    next.w_next = om;
+    commit_scalars(next, sum[0].x, sum[1], (d.flags & MPA_SOLVE_REF_LOOP) != 0);
+    const bool go = !next.done && !next.restart_pending;
+    if (go) {  // k_update_p of the next iteration
+        const double2 beta = cmul(cdiv(next.rho_next, next.rho), cdiv(next.alpha, next.w));
+        const C bt = from_d<T>(beta);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int i = index(e);
+            if (i >= 0) p[i] = cadd(st[e], cmul(bt, csub(p[i], cmul(wt, v[i]))));
+        }
+    }
+    if (threadIdx.x == 0) {
+        next.p_ready = go ? 1 : 0;
+        *sc = next;
     }
 }
 
@@ -339,6 +494,7 @@ struct Plan {
     std::vector<int2> mv_work[kTileClasses];  // (job, row block) per tile class; same for every job set
     std::vector<MfJob> mf_ps, mf_st, mf_xt;   // matrix-free systems (launched by value)
     bool any_precond = false;
+    bool half = false;  // the half-iteration kernels serve this plan
     // device copies
     SysDev* d_sys = nullptr;
     int3* d_vec = nullptr;
@@ -441,6 +597,9 @@ int build_plan(Plan& P, int nsys, const mpa_system* S_, int dtype, void* scratch
         std::vector<int2>& mw = P.mv_work[gemv_class(S)];
         for (int b = 0; b < rb; b++) mw.push_back(make_int2(i, b));
     }
+    int maxn = 0;
+    for (int i = 0; i < nsys; i++) maxn = std::max(maxn, S_[i].n);
+    P.half = !P.any_precond && maxn <= kHalfMaxN;
     for (auto& w : P.mv_work) order_work_longest_first(w, [&](int i) { return S_[i].n; });
     char* p = (char*)scratch;
     P.d_sys = (SysDev*)p; p += align256(sizeof(SysDev) * nsys);
@@ -517,9 +676,30 @@ int launch_start(const Plan& P, hipStream_t st) {
     return MPA_OK;
 }
 
+// The direction p of the first iteration (or of the first after a restart),
+// which the half-iteration kernels expect; systems that have theirs keep it.
+template <typename T>
+int launch_direction(const Plan& P, hipStream_t st) {
+    if (!P.half) return MPA_OK;  // formed at the start of every iteration
+    hipLaunchKernelGGL(k_update_p<T>, dim3((unsigned)P.vec_work.size()), dim3(kThreads), 0, st, P.d_sys, P.d_vec);
+    MPA_LAUNCH_CHECK();
+    return MPA_OK;
+}
+
 template <typename T>
 int launch_iteration(const Plan& P, hipStream_t st) {
     const int nv = (int)P.vec_work.size(), ns = (int)P.scal_work.size();
+    if (P.half) {
+        const dim3 g(ns), t(kHalfT);
+        int rc = matvec_phase<T>(P, P.d_mv_ps, P.mf_ps, st);
+        if (rc) return rc;
+        hipLaunchKernelGGL(k_half1<T>, g, t, 0, st, P.d_sys, P.d_scal);
+        rc = matvec_phase<T>(P, P.d_mv_st, P.mf_st, st);
+        if (rc) return rc;
+        hipLaunchKernelGGL(k_half2<T>, g, t, 0, st, P.d_sys, P.d_scal);
+        MPA_LAUNCH_CHECK();
+        return MPA_OK;
+    }
     hipLaunchKernelGGL(k_update_p<T>, dim3(nv), dim3(kThreads), 0, st, P.d_sys, P.d_vec);
     if (P.any_precond) hipLaunchKernelGGL(k_precond<T>, dim3(nv), dim3(kThreads), 0, st, P.d_sys, P.d_vec, 0);
     int rc = matvec_phase<T>(P, P.d_mv_ps, P.mf_ps, st);
@@ -582,9 +762,6 @@ struct IterGraph {
         if (graph) (void)hipGraphDestroy(graph);
     }
 };
-
-template <typename T>
-int launch_iteration(const Plan& P, hipStream_t st);
 
 template <typename T>
 int capture_iterations(const Plan& P, int k, IterGraph& g) {
@@ -655,7 +832,7 @@ int solve_batch(int nsys, const mpa_system* S_, void* scratch, int* iters, doubl
     int rounds = std::max(1, std::min(4, maxit) / k_sync);
     bool from_start = maxit > 0;  // the decay so far is measured from iteration 0
     for (int i = 0; i < nsys; i++) from_start &= (S_[i].flags & MPA_SOLVE_REF_LOOP) == 0;  // x0 = b: restart first
-    if (from_start && (rc = launch_rounds(rounds))) return rc;
+    if (from_start && ((rc = launch_direction<T>(P, st)) || (rc = launch_rounds(rounds)))) return rc;
     for (;;) {
         rc = read_scalars(P, host, st, noalloc);
         if (rc) return rc;
@@ -666,7 +843,7 @@ int solve_batch(int nsys, const mpa_system* S_, void* scratch, int* iters, doubl
         }
         if (any_restart) {
             rc = launch_restart<T>(P, st);
-            if (rc) return rc;
+            if (rc || (rc = launch_direction<T>(P, st))) return rc;
             prev_r2.clear();
             from_start = false;
             rounds = 1;
@@ -841,6 +1018,10 @@ int mpa_systems_advance(int nsys, const mpa_system* systems, int dtype, void* sc
     for (const Scal& c : host) restart |= c.restart_pending != 0;
     if (restart) {
         rc = dtype == MPA_C128 ? launch_restart<double>(P, st) : launch_restart<float>(P, st);
+        if (rc) return rc;
+    }
+    if (iterations > 0) {
+        rc = dtype == MPA_C128 ? launch_direction<double>(P, st) : launch_direction<float>(P, st);
         if (rc) return rc;
     }
     for (int k = 0; k < iterations; k++) {

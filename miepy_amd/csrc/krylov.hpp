@@ -17,7 +17,8 @@ struct Scal {
     double2 rho_next, alpha_next, w_next;
     double r0_sq, rhs_sq, rnorm2, tol2;
     int it, done, status, restarts;
-    int maxiter, restart_pending, init_pending, pad1;  // init_pending: x0 = b, r = b - A b not yet formed
+    int maxiter, restart_pending, init_pending;  // init_pending: x0 = b, r = b - A b not yet formed
+    int p_ready;  // p already holds the next iteration's direction (formed by k_half2)
 };
 
 // One linear system (I + T) x = b with S right-hand sides, as the kernels see it.

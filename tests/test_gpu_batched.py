@@ -258,3 +258,24 @@ def test_batched_assembly_equals_single(dev):
         assert np.array_equal(out.cpu().numpy(), ref[0].cpu().numpy()), q
         if out32 is not None:
             assert np.array_equal(out32.cpu().numpy(), ref[1].cpu().numpy()), q
+
+
+@pytest.mark.parametrize("c64", [False, True])
+def test_solo_small_system_equals_batch_with_a_large_one(dev, c64):
+    """A batch whose largest system exceeds 4096 unknowns runs its vector work
+    in other kernels than a small system alone: every system's iterates are
+    the same, bit for bit, at n on both sides of a 1024-element group and at
+    the largest size of the one-workgroup kernels."""
+    import torch
+    dtype, tol = (dev.C64, 1e-5) if c64 else (dev.C128, 1e-11)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    mats, rhs = [], []
+    for n, S in ((2, 1), (254, 3), (1024, 1), (1026, 2), (3000, 1), (4096, 5), (4200, 1)):
+        A = torch.randn((n, n), dtype=dtype, device="cuda", generator=g) * (0.3 / n ** 0.5)
+        mats.append(A + torch.eye(n, dtype=dtype, device="cuda"))
+        rhs.append(torch.randn((S, n), dtype=dtype, device="cuda", generator=g))
+    xs, reps = dev.bicgstab_batched(mats, rhs, tol=tol, maxiter=300)
+    for A, b, x, rep in zip(mats, rhs, xs, reps):
+        x1, rep1 = dev.bicgstab(A, b, tol=tol, maxiter=300)
+        assert rep.converged and rep.iterations == rep1.iterations
+        assert torch.equal(x, x1)
