@@ -750,6 +750,20 @@ int read_scalars(const Plan& P, std::vector<Scal>& out, hipStream_t st, bool noa
     return MPA_OK;
 }
 
+// Whether a plan's iterations are replayed from a graph (MPA_OPT_GRAPHS 2:
+// always, 0: never).  A replayed kernel starts about 1 us later than an eager
+// one and the capture costs each solve some 60 us, so eager launches win as
+// long as the host keeps ahead of the GPU: n = 592 33.2 us per iteration
+// replayed and 27.9 eager, a batch of 12 clusters 27.5 and 26.6 ms, 1000
+// spheres matrix-free 9.5 and 9.05 ms.  Many matrix-free systems, each with
+// its own launches, turn that around: 24 clusters 12.3 ms replayed and 13.3
+// eager, 64 clusters 34.2 and 37.0.
+constexpr size_t kGraphMatfree = 16;
+bool graphs_pay(const Plan& P) {
+    const int opt = mpa_option(MPA_OPT_GRAPHS);
+    return opt == 2 || (opt != 0 && P.mf_ps.size() >= kGraphMatfree);
+}
+
 // k BiCGSTAB iterations of a plan recorded once as a HIP graph and replayed.
 struct IterGraph {
     hipGraph_t graph = nullptr;
@@ -801,7 +815,7 @@ int solve_batch(int nsys, const mpa_system* S_, void* scratch, int* iters, doubl
     std::vector<Scal> host;
     long launched = 0;
     IterGraph graph;
-    const bool use_graph = !noalloc && mpa_option(MPA_OPT_GRAPHS) != 0 && !mpa_profile_active();
+    const bool use_graph = !noalloc && graphs_pay(P) && !mpa_profile_active();
     if (use_graph) {
         rc = capture_iterations<T>(P, k_sync, graph);
         if (rc) return rc;

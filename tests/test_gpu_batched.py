@@ -279,3 +279,34 @@ def test_solo_small_system_equals_batch_with_a_large_one(dev, c64):
         x1, rep1 = dev.bicgstab(A, b, tol=tol, maxiter=300)
         assert rep.converged and rep.iterations == rep1.iterations
         assert torch.equal(x, x1)
+
+
+@pytest.mark.parametrize("sync_every", [1, 3])
+def test_forced_graph_replay_equals_eager(dev, sync_every):
+    """MPA_OPT_GRAPHS 2 replays every solve from graphs, whatever its size:
+    stored and matrix-free systems below and above 4096 unknowns give the
+    eager launches' results bit for bit."""
+    import torch
+    import miepy_amd._lib as L
+    lib = L.load()
+    systems = _systems(dev, seed=4, count=3)
+    g = torch.Generator(device="cuda").manual_seed(6)
+    big = torch.randn((4200, 4200), dtype=dev.C128, device="cuda", generator=g) * 0.004
+    big += torch.eye(4200, dtype=dev.C128, device="cuda")
+    mats = [dev.assemble(pos, ms, k, add_identity=True) for pos, ms, k, _ in systems]
+    ops = [dev.ClusterOperator(pos, ms, k, max_rhs=b.shape[0]) for pos, ms, k, b in systems]
+    bs = [dev.to_device(b, dev.C128) for *_, b in systems]
+    b_big = torch.randn((2, 4200), dtype=dev.C128, device="cuda", generator=g)
+    saved = lib.mpa_get_option(L.MPA_OPT_GRAPHS)
+    out = {}
+    try:
+        for mode in (2, 0):
+            assert lib.mpa_set_option(L.MPA_OPT_GRAPHS, mode) == 0
+            out[mode] = []
+            for ms, rhs in ((mats, bs), (mats + [big], bs + [b_big]), (ops, bs)):
+                xs, reps = dev.bicgstab_batched(ms, rhs, tol=1e-10, maxiter=500, sync_every=sync_every)
+                out[mode] += list(zip(xs, [r.iterations for r in reps]))
+    finally:
+        lib.mpa_set_option(L.MPA_OPT_GRAPHS, saved)
+    for (xg, ig), (xe, ie) in zip(out[2], out[0]):
+        assert ig == ie and torch.equal(xg, xe)
