@@ -258,13 +258,20 @@ int launch_assembly(int N, int lmax, const double* positions, const double* mie,
 // forms the product entry by entry for every pair inside an n x n scratch
 // matrix).  Here the bare X blocks are assembled in place (unit Mie
 // coefficients) and every column block is then multiplied on the right by
-// its particle's T-matrix: one workgroup per (column block j, 32 rows)
-// stages the old 32 x bs values and (bs <= 48) Tm_j in LDS, forms the
-// products in FP64 and writes the block back; the identity is added on the
-// diagonal blocks (which are zero before the product).
+// its particle's T-matrix on the FP64 matrix cores, as a real product: K
+// position 2q + odd holds Re or Im of X[.][q], real column 2c + part of the
+// right operand Re or Im of the product (Re T, -Im T / Im T, Re T).  A
+// workgroup owns one column block and kApplyRows rows: Tm_j stays in LDS as
+// the right operand, each wave takes 16 rows at a time through its own part of
+// LDS (coalesced in, operand layout out) and writes their products back; the
+// identity is added on the diagonal blocks (which are zero before the
+// product).  110 particles at lmax 3 (174 MB): 187 us with one thread per
+// entry, which read two LDS values per multiply-add, 96 us so.
 
-constexpr int kApplyRows = 32;
-constexpr int kApplyTmLdsMax = 48;  // bs up to which Tm_j is staged in LDS (lmax <= 4)
+typedef double ad4 __attribute__((ext_vector_type(4)));
+
+constexpr int kApplyRows = 256;  // rows of a workgroup
+constexpr int kApplyWaves = kThreads / 64;
 
 template <typename OutT>
 __device__ inline double2 load_c(const OutT* p);
@@ -278,34 +285,86 @@ __device__ inline double2 load_c<float2>(const float2* p) {
     return make_double2(v.x, v.y);
 }
 
-template <typename OutT>
-__global__ __launch_bounds__(kThreads) void k_apply_tmatrix(int N, int bs, int nrowblocks,
-                                                             const double2* __restrict__ tm, int add_identity,
-                                                             OutT* __restrict__ out) {
-    extern __shared__ double2 lds[];
+// LDS: Tm_j [bs][bs + 1] (up to lmax 5; read through the caches above), then per wave 16 rows of X [bs + 1]
+template <typename OutT, int LMAX>
+__global__ __launch_bounds__(kThreads) void k_apply_tmatrix(int N, int nrowblocks, const double2* __restrict__ tm,
+                                                             int add_identity, OutT* __restrict__ out) {
+    constexpr int bs = 2 * LMAX * (LMAX + 2), ls = bs + 1, NT = (bs + 7) / 8;
+    constexpr bool staged = LMAX <= 5;
+    __shared__ double2 X_[kApplyWaves * 16 * ls];
+    __shared__ double2 T_[staged ? bs * ls : 1];
     const int j = blockIdx.x / nrowblocks;
     const int r0 = (blockIdx.x % nrowblocks) * kApplyRows;
     const size_t n = (size_t)bs * N;
     const int nr = (int)min((size_t)kApplyRows, n - r0);
-    double2* old = lds;                         // [kApplyRows][bs]
-    double2* tml = old + kApplyRows * bs;       // [bs][bs] when staged
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, g = lane >> 4, col = lane & 15;
+    const int part = col & 1, odd = g & 1;
+    double2* X = X_ + w * 16 * ls;
     const double2* tmj = tm + (size_t)j * bs * bs;
-    const bool staged = bs <= kApplyTmLdsMax;
-    for (int u = threadIdx.x; u < nr * bs; u += kThreads) {
-        const int rr = u / bs, c = u - rr * bs;
-        old[u] = load_c<OutT>(out + (size_t)(r0 + rr) * n + (size_t)j * bs + c);
+    if (staged) {
+        for (int u = threadIdx.x; u < bs * bs; u += kThreads) T_[(u / bs) * ls + u % bs] = tmj[u];
+        __syncthreads();
     }
-    if (staged)
-        for (int u = threadIdx.x; u < bs * bs; u += kThreads) tml[u] = tmj[u];
-    __syncthreads();
-    const double2* T = staged ? tml : tmj;
-    for (int u = threadIdx.x; u < nr * bs; u += kThreads) {
-        const int rr = u / bs, c = u - rr * bs;
-        double2 acc = make_double2(0.0, 0.0);
-        for (int q = 0; q < bs; q++) cfma(acc, old[rr * bs + q], T[q * bs + c]);
-        const size_t row = (size_t)r0 + rr;
-        if (add_identity && row == (size_t)j * bs + c) acc.x += 1.0;
-        store<OutT>(out + row * n + (size_t)j * bs + c, acc);
+    OutT* block = out + (size_t)r0 * n + (size_t)j * bs;
+    constexpr int total = 16 * bs;
+    // the next 16 rows are read while the current ones are multiplied
+    constexpr int LD = total / 64 + (total % 64 ? 1 : 0);
+    double2 v[LD];
+    auto load = [&](int t0) {
+#pragma unroll
+        for (int e = 0; e < LD; e++) {
+            const int u = min(64 * e + lane, total - 1), rr = u / bs, c = u - rr * bs;
+            v[e] = load_c<OutT>(block + (size_t)min(t0 + rr, nr - 1) * n + c);
+        }
+    };
+    if (w * 16 < nr) load(w * 16);
+    for (int t0 = w * 16; t0 < nr; t0 += 16 * kApplyWaves) {
+#pragma unroll
+        for (int e = 0; e < LD; e++) {
+            const int u = 64 * e + lane, rr = u / bs, c = u - rr * bs;
+            if (u < total) X[rr * ls + c] = v[e];
+        }
+        if (t0 + 16 * kApplyWaves < nr) load(t0 + 16 * kApplyWaves);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        ad4 acc[NT];
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) acc[t][q] = 0.0;
+        for (int s = 0; s < bs / 2; s++) {  // 4 real K positions: complex q = 2 s, 2 s + 1 (bs is even)
+            const int q = 2 * s + (g >> 1);
+            const double2 xv = X[col * ls + q];
+            const double a = odd ? xv.y : xv.x;
+#pragma unroll
+            for (int t = 0; t < NT; t++) {
+                const int c = min(8 * t + (col >> 1), bs - 1);
+                const double2 u = staged ? T_[q * ls + c] : tmj[q * bs + c];
+                const double b = odd ? (part ? u.x : -u.y) : (part ? u.y : u.x);
+                acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc[t], 0, 0, 0);
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        double* Xd = (double*)X;
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+            const int c = 8 * t + (col >> 1);
+            if (c < bs)
+#pragma unroll
+                for (int q = 0; q < 4; q++) Xd[2 * ((4 * q + g) * ls + c) + part] = acc[t][q];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        for (int u = lane; u < total; u += 64) {
+            const int rr = u / bs, c = u - rr * bs;
+            if (t0 + rr >= nr) continue;
+            double2 v = X[rr * ls + c];
+            if (add_identity && (size_t)(r0 + t0 + rr) == (size_t)j * bs + c) v.x += 1.0;
+            store<OutT>(block + (size_t)(t0 + rr) * n + c, v);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
     }
 }
 
@@ -319,9 +378,12 @@ int launch_apply_tmatrix(int N, int lmax, const double* tmatrix, int add_identit
         mpa_set_error("particle_aggregate_tmatrix: N=%d too large for one launch", N);
         return MPA_ERR_ARG;
     }
-    const size_t lds = sizeof(double2) * ((size_t)kApplyRows * bs + (bs <= kApplyTmLdsMax ? (size_t)bs * bs : 0));
-    hipLaunchKernelGGL(k_apply_tmatrix<OutT>, dim3((unsigned)nblocks), dim3(kThreads), lds, s, N, bs, nrb,
-                       (const double2*)tmatrix, add_identity, out);
+#define MPA_APPLY(L_)                                                                                               \
+    if (lmax == L_)                                                                                                 \
+        hipLaunchKernelGGL((k_apply_tmatrix<OutT, L_>), dim3((unsigned)nblocks), dim3(kThreads), 0, s, N, nrb,      \
+                           (const double2*)tmatrix, add_identity, out);
+    MPA_APPLY(1) MPA_APPLY(2) MPA_APPLY(3) MPA_APPLY(4) MPA_APPLY(5) MPA_APPLY(6)
+#undef MPA_APPLY
     MPA_LAUNCH_CHECK();
     return MPA_OK;
 }

@@ -128,3 +128,20 @@ def test_cluster_dense_tmatrices_match_oracle_lu(dev, oracle, mode):
     assert np.linalg.norm(cl.p_inc - p_inc) <= 1e-9 * np.linalg.norm(p_inc)
     p_scat = np.einsum("naibj,nbj->nai", tm, p_inc)
     assert np.linalg.norm(cl.p_scat - p_scat) <= 1e-9 * np.linalg.norm(p_scat)
+
+
+@pytest.mark.parametrize("N,lmax", [(1, 1), (43, 1), (17, 2), (18, 3), (6, 4), (4, 5), (3, 6)])
+def test_particle_aggregate_row_blocks(dev, oracle, N, lmax):
+    """The T-matrix product at row counts below, at and above one workgroup's
+    256 rows and with a partial last group of 16, every order up to 6 (6: the
+    T-matrix is read past LDS): the bars of the oracle test above."""
+    pos, rng = _geometry(N, 90 + N)
+    k = 2 * np.pi / (600 * nm)
+    tm = _random_tmatrices(rng, N, lmax)
+    ref = oracle.particle_aggregate_tmatrix(pos, tm, k)
+    ref = ref + np.eye(ref.shape[0])
+    scale = np.abs(ref).max()
+    got = dev.assemble_tmatrix(pos, tm, k, add_identity=True).cpu().numpy()
+    assert np.max(np.abs(got - ref)) <= 1e-12 * scale
+    got32 = dev.assemble_tmatrix(pos, tm, k, add_identity=True, dtype=dev.C64).cpu().numpy()
+    assert np.max(np.abs(got32 - ref)) <= 1e-6 * scale
