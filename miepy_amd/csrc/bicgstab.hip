@@ -258,26 +258,42 @@ __device__ __forceinline__ void commit_scalars(Scal& c, double rr, double2 r0r, 
     }
 }
 
-// commit the iteration's scalars
-__global__ __launch_bounds__(kThreads) void k_commit(const SysDev* __restrict__ sys, const int2* __restrict__ cw) {
-    const int2 c2 = cw[blockIdx.x];
-    const SysDev& d = sys[c2.x];
-    const int s = c2.y;
-    Scal& c = glob(d.scal)[s];
-    if (c.done || c.restart_pending) return;
+// Commit the iteration's scalars and form the next direction (k_update_p) in
+// one launch.  Every workgroup of a right-hand side computes the same new
+// scalars from the old ones; the last to have read the old ones (counted in
+// steps of 2 in p_ready, which is 0 here) writes the new ones.  No workgroup
+// waits for another.
+template <typename T>
+__global__ __launch_bounds__(kThreads) void k_commit_p(const SysDev* __restrict__ sys, const int3* __restrict__ work) {
+    using C = cplx_t<T>;
+    VEC_PROLOGUE
+    Scal* sc = glob(d.scal) + s;
+    Scal next = *sc;
+    if (next.done || next.restart_pending) return;
     const double2 rr = reduce_partials(d.part, d.G, s, 3);
     const double2 r0r = reduce_partials(d.part, d.G, s, 4);
-    if (threadIdx.x == 0) {
-        Scal next = c;
-        commit_scalars(next, rr.x, r0r, (d.flags & MPA_SOLVE_REF_LOOP) != 0);
-        c = next;
+    commit_scalars(next, rr.x, r0r, (d.flags & MPA_SOLVE_REF_LOOP) != 0);
+    const bool go = !next.done && !next.restart_pending;
+    if (go) {
+        const double2 beta = cmul(cdiv(next.rho_next, next.rho), cdiv(next.alpha, next.w));
+        const C bt = from_d<T>(beta), wt = from_d<T>(next.w);
+        C *p = glob((C*)d.p), *r = glob((C*)d.r), *v = glob((C*)d.v);
+        for (int i = g * kThreads + threadIdx.x; i < n; i += stride) {
+            const size_t k = base + i;
+            p[k] = cadd(r[k], cmul(bt, csub(p[k], cmul(wt, v[k]))));
+        }
+    }
+    __syncthreads();  // this workgroup's reads of the old scalars are done
+    if (threadIdx.x == 0 && atomicAdd(&sc->p_ready, 2) == 2 * (d.G - 1)) {
+        next.p_ready = go ? 1 : 0;
+        *sc = next;
     }
 }
 
 // ---- the vector work of a half iteration in one workgroup per (system, RHS) ------
 //
 // Up to kHalfMaxN unknowns one workgroup per right-hand side does what the
-// kernels above do in two and four launches, whose fixed 4-5 us each were most
+// kernels above do in two and three launches, whose fixed 4-5 us each were most
 // of a small solve's time: k_half1 <r0, v>, alpha and s; k_half2 <t, s>, <t, t>,
 // w, x, r, ||r||^2, <r0, r>, the commit and the next direction p.  The sums are
 // taken in the same order as there: element i = g 256 + t + k G 256 belongs to
@@ -676,11 +692,10 @@ int launch_start(const Plan& P, hipStream_t st) {
     return MPA_OK;
 }
 
-// The direction p of the first iteration (or of the first after a restart),
-// which the half-iteration kernels expect; systems that have theirs keep it.
+// The direction p of the first iteration (or of the first after a restart): an
+// iteration expects it and forms the next one; systems that have theirs keep it.
 template <typename T>
 int launch_direction(const Plan& P, hipStream_t st) {
-    if (!P.half) return MPA_OK;  // formed at the start of every iteration
     hipLaunchKernelGGL(k_update_p<T>, dim3((unsigned)P.vec_work.size()), dim3(kThreads), 0, st, P.d_sys, P.d_vec);
     MPA_LAUNCH_CHECK();
     return MPA_OK;
@@ -700,7 +715,6 @@ int launch_iteration(const Plan& P, hipStream_t st) {
         MPA_LAUNCH_CHECK();
         return MPA_OK;
     }
-    hipLaunchKernelGGL(k_update_p<T>, dim3(nv), dim3(kThreads), 0, st, P.d_sys, P.d_vec);
     if (P.any_precond) hipLaunchKernelGGL(k_precond<T>, dim3(nv), dim3(kThreads), 0, st, P.d_sys, P.d_vec, 0);
     int rc = matvec_phase<T>(P, P.d_mv_ps, P.mf_ps, st);
     if (rc) return rc;
@@ -711,7 +725,7 @@ int launch_iteration(const Plan& P, hipStream_t st) {
     if (rc) return rc;
     hipLaunchKernelGGL(k_dot_ts<T>, dim3(nv), dim3(kThreads), 0, st, P.d_sys, P.d_vec);
     hipLaunchKernelGGL(k_update_xr<T>, dim3(nv), dim3(kThreads), 0, st, P.d_sys, P.d_vec);
-    hipLaunchKernelGGL(k_commit, dim3(ns), dim3(kThreads), 0, st, P.d_sys, P.d_scal);
+    hipLaunchKernelGGL(k_commit_p<T>, dim3(nv), dim3(kThreads), 0, st, P.d_sys, P.d_vec);
     MPA_LAUNCH_CHECK();
     return MPA_OK;
 }

@@ -18,7 +18,7 @@ struct Scal {
     double r0_sq, rhs_sq, rnorm2, tol2;
     int it, done, status, restarts;
     int maxiter, restart_pending, init_pending;  // init_pending: x0 = b, r = b - A b not yet formed
-    int p_ready;  // p already holds the next iteration's direction (formed by k_half2)
+    int p_ready;  // 1: p already holds the next iteration's direction (formed with the commit)
 };
 
 // One linear system (I + T) x = b with S right-hand sides, as the kernels see it.
