@@ -670,7 +670,6 @@ __global__ __launch_bounds__(kT) void k_lu_diag_solve(const double2* __restrict_
     double2* xs = x + (size_t)blockIdx.x * n + b0;
     double2 y = q < nb ? xs[q] : make_double2(0.0, 0.0);
     const double2 inv = !LOWER && q < nb ? cdiv(make_double2(1.0, 0.0), B[q][q]) : make_double2(1.0, 0.0);
-#pragma unroll 4
     for (int k = 0; k < nb; k++) {
         const int r = LOWER ? k : nb - 1 - k;
         const double2 b = B[q][r];
