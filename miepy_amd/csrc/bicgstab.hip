@@ -843,7 +843,16 @@ int solve_batch(int nsys, const mpa_system* S_, void* scratch, int* iters, doubl
     // a few dozen iterations reads its scalars back a handful of times.
     std::vector<double> prev_r2;
     std::vector<int> prev_it;
+    // Every iteration leaves the next one's direction behind; the first is formed
+    // here unless a restart has already done so (k_update_p before an iteration
+    // must run once: a second call would apply beta again).
+    bool have_direction = false;
     auto launch_rounds = [&](int nr) -> int {
+        if (!have_direction) {
+            const int r1 = launch_direction<T>(P, st);
+            if (r1) return r1;
+            have_direction = true;
+        }
         for (int round = 0; round < nr; round++) {
             if (use_graph) {
                 MPA_HIP_CHECK(hipGraphLaunch(graph.exec, st));
@@ -860,7 +869,7 @@ int solve_batch(int nsys, const mpa_system* S_, void* scratch, int* iters, doubl
     int rounds = std::max(1, std::min(4, maxit) / k_sync);
     bool from_start = maxit > 0;  // the decay so far is measured from iteration 0
     for (int i = 0; i < nsys; i++) from_start &= (S_[i].flags & MPA_SOLVE_REF_LOOP) == 0;  // x0 = b: restart first
-    if (from_start && ((rc = launch_direction<T>(P, st)) || (rc = launch_rounds(rounds)))) return rc;
+    if (from_start && (rc = launch_rounds(rounds))) return rc;
     for (;;) {
         rc = read_scalars(P, host, st, noalloc);
         if (rc) return rc;
@@ -872,6 +881,7 @@ int solve_batch(int nsys, const mpa_system* S_, void* scratch, int* iters, doubl
         if (any_restart) {
             rc = launch_restart<T>(P, st);
             if (rc || (rc = launch_direction<T>(P, st))) return rc;
+            have_direction = true;
             prev_r2.clear();
             from_start = false;
             rounds = 1;

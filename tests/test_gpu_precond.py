@@ -203,3 +203,26 @@ def test_complex64_preconditioned(dev):
     assert rep.converged
     ref = np.linalg.solve(A, b)
     assert np.linalg.norm(x.cpu().numpy().reshape(-1) - ref) <= 1e-4 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("n", [512, 4200])
+@pytest.mark.parametrize("bad", ["zero", "nan", "zero and nan"])
+def test_plain_system_beside_finished_reference_loops(dev, n, bad):
+    """A reference-loop system whose right-hand sides are all zero or not
+    finite is done before the first iteration and never restarts; the plain
+    system beside it still gets its first direction: its iterates equal its
+    own solve's bit for bit, in the one-workgroup vector kernels and past
+    their 4096 unknowns."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(n)
+    A = torch.randn((n, n), dtype=dev.C128, device="cuda", generator=g) * (0.3 / n ** 0.5)
+    A += torch.eye(n, dtype=dev.C128, device="cuda")
+    b = torch.randn((2, n), dtype=dev.C128, device="cuda", generator=g)
+    b_ref = torch.zeros((2, n), dtype=dev.C128, device="cuda")
+    if bad != "zero":
+        b_ref[1 if bad == "zero and nan" else slice(None), 3] = float("nan")
+    xs, reps = dev.bicgstab_batched([A, A], [b_ref, b], tol=1e-10, maxiter=200, ref_loop=[True, False])
+    x1, rep1 = dev.bicgstab(A, b, tol=1e-10, maxiter=200)
+    assert rep1.converged and reps[1].converged and reps[1].iterations == rep1.iterations
+    assert torch.equal(xs[1], x1)
+    assert list(reps[0].iterations) == [0, 0]
