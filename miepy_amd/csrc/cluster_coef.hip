@@ -67,23 +67,29 @@ __global__ __launch_bounds__(kCT) void k_cluster_coef(int N, int L, int lmax_in,
         ur[e] = u < total ? u % rmax_out : 0;
         acc0[e] = acc1[e] = make_double2(0, 0);
     }
+    // One test for both uses: special functions are formed for exactly the
+    // particles whose coefficients are read (a NaN distance is not the origin).
+    auto at_origin = [&](int i, double& dx, double& dy, double& dz) {
+        dx = ox - pos[3 * i];
+        dy = oy - pos[3 * i + 1];
+        dz = oz - pos[3 * i + 2];
+        return (dx == 0.0 && dy == 0.0 && dz == 0.0) || sqrt(dx * dx + dy * dy + dz * dz) < origin_tol;
+    };
     for (int i0 = blockIdx.x; i0 < N; i0 += kCoefGroup * gridDim.x) {
         __syncthreads();  // the previous group's HL is no longer read
         {
             const int g = threadIdx.x >> 4, mu = threadIdx.x & 15, i = i0 + g * (int)gridDim.x;
-            if (g < kCoefGroup && i < N && mu <= 2 * L + 1) {
-                const double dx = ox - pos[3 * i], dy = oy - pos[3 * i + 1], dz = oz - pos[3 * i + 2];
-                if (sqrt(dx * dx + dy * dy + dz * dz) > 0.0) pair_hl(HL[g], eph[g], mu, L, dx, dy, dz, k, 2);
-            }
+            double dx, dy, dz;
+            if (g < kCoefGroup && i < N && mu <= 2 * L + 1 && !at_origin(i, dx, dy, dz))
+                pair_hl(HL[g], eph[g], mu, L, dx, dy, dz, k, 2);
         }
         for (int g = 0; g < kCoefGroup; g++) {
             const int i = i0 + g * (int)gridDim.x;
             if (i >= N) break;
-            const double dx = ox - pos[3 * i], dy = oy - pos[3 * i + 1], dz = oz - pos[3 * i + 2];
-            const bool at_origin = (dx == 0.0 && dy == 0.0 && dz == 0.0) ||
-                                   sqrt(dx * dx + dy * dy + dz * dz) < origin_tol;
+            double dx, dy, dz;
+            const bool here = at_origin(i, dx, dy, dz);
             __syncthreads();  // HL is written (g = 0); the previous particle's XA, XB are read
-            if (!at_origin)
+            if (!here)
                 for (int q = threadIdx.x; q < pairs; q += kCT) {
                     const int r = q / rmax_in, rp = q - r * rmax_in;
                     tuple_xab(tab, r * rmaxL + rp, HL[g], eph[g], XA[q], XB[q]);
@@ -95,7 +101,7 @@ __global__ __launch_bounds__(kCT) void k_cluster_coef(int N, int L, int lmax_in,
                 if (us[e] < 0) continue;
                 const int r = ur[e];
                 const double2* ps = p_scat + ((size_t)us[e] * N + i) * 2 * rmax_in;
-                if (at_origin) {
+                if (here) {
                     if (r < rmax_in) {
                         const int v = mode_n(r);
                         acc0[e] = cadd(acc0[e], mi ? cmul(mi[v - 1], ps[r]) : ps[r]);

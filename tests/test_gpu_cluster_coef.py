@@ -62,6 +62,29 @@ def test_particle_at_origin_truncates(dev):
     assert np.allclose(both - other, p[0, 0, :, :8], rtol=0, atol=1e-13 * np.abs(both).max())
 
 
+@pytest.mark.parametrize("coord,tiny", [((np.nan, 0.3, 0.2), False), ((1.0, np.inf, 0.2), False), ((1e-200, 0.0, 0.0), True)])
+@pytest.mark.parametrize("N,at", [(1, 0), (6, 4), (140, 131)])
+def test_positions_without_a_distance_give_nan(dev, coord, tiny, N, at):
+    """A particle whose distance from the origin is NaN, infinite or underflows
+    to zero without its being at the origin has no translation coefficients:
+    every output is NaN, never a sum of other particles' special functions
+    (groups of four particles share a workgroup's LDS; 140 particles: more
+    than the 128 workgroups).  In the cluster T-matrix a distance below 1e-15
+    counts as the origin, so there the underflowing one stays finite."""
+    rng = np.random.default_rng(N)
+    pos = rng.uniform(-3, 3, size=(N, 3))
+    p = rng.normal(size=(2, N, 2, 8)) + 1j * rng.normal(size=(2, N, 2, 8))
+    good = dev.cluster_coefficients(pos, p, 6.0, np.zeros(3), 3).cpu().numpy()
+    assert np.isfinite(good).all()
+    pos[at] = coord
+    got = dev.cluster_coefficients(pos, p, 6.0, np.zeros(3), 3).cpu().numpy()
+    assert np.isnan(got).all()
+    mie = dev.to_device(rng.normal(size=(N, 2, 2)) + 0j, dev.C128)
+    X = dev.to_device(rng.normal(size=(30, N * 16)) + 0j, dev.C128)
+    T = dev.cluster_tmatrix(pos, mie, X, 6.0, np.zeros(3), 3).cpu().numpy()
+    assert np.isfinite(T).all() if tiny else np.isnan(T).all()
+
+
 def test_cluster_cross_sections_match_oracle(dev, oracle):
     rng = np.random.default_rng(5)
     for lmax in (1, 3, 6):
