@@ -149,8 +149,8 @@ __device__ inline void gemv_rows(const MvDev& J, int first, int end) {
 // step of its 16 rows and of the right-hand sides from global memory into
 // registers in runs of 64 Q bytes per row, one step ahead, and through its own
 // part of LDS into the MFMA operand layout; nothing is shared between waves,
-// so the loop has no barriers.  At the end the waves' tiles are added in LDS
-// in wave order.  Rows of an LDS buffer are padded by 16 bytes: the 16 rows of
+// so the loop has no barriers.  At the end the waves' tiles are added in LDS.
+// Rows of an LDS buffer are padded by 16 bytes: the 16 rows of
 // one operand read then cover all banks.
 //   A operand: lane l holds row l % 16 and, per 16-byte read, 4 consecutive
 //     reals of c64 (2 complex) or 2 of c128 (1 complex) at the K offset of
@@ -168,22 +168,32 @@ template <typename T> struct MfmaTile;
 template <> struct MfmaTile<float> {
     using acc = fvec4;
     static constexpr int C = 2;  // complex entries per 16-byte load
+    static constexpr int K = 4;  // MFMAs per 16-byte load of A
     __device__ static int row(int g, int i) { return 4 * g + i; }
-    // the 4 K positions of one 16-byte load of A times X'
-    __device__ static void fma(acc& d, fvec4 a, fvec4 x, int part) {
-        d = __builtin_amdgcn_mfma_f32_16x16x4f32(a[0], part ? x.y : x.x, d, 0, 0, 0);
-        d = __builtin_amdgcn_mfma_f32_16x16x4f32(a[1], part ? x.x : -x.y, d, 0, 0, 0);
-        d = __builtin_amdgcn_mfma_f32_16x16x4f32(a[2], part ? x.w : x.z, d, 0, 0, 0);
-        d = __builtin_amdgcn_mfma_f32_16x16x4f32(a[3], part ? x.z : -x.w, d, 0, 0, 0);
+    // the K MFMAs of one 16-byte load of A times X', number e into chain (c0 + e) % NC
+    template <int NC>
+    __device__ static void fma(acc (&d)[NC], int c0, fvec4 a, fvec4 x, int part) {
+        const float b[K] = {part ? x.y : x.x, part ? x.x : -x.y, part ? x.w : x.z, part ? x.z : -x.w};
+#pragma unroll
+        for (int e = 0; e < K; e++) {
+            acc& s = d[(c0 + e) % NC];
+            s = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], s, 0, 0, 0);
+        }
     }
 };
 template <> struct MfmaTile<double> {
     using acc = d4v;
     static constexpr int C = 1;
+    static constexpr int K = 2;
     __device__ static int row(int g, int i) { return 4 * i + g; }
-    __device__ static void fma(acc& d, dvec2 a, dvec2 x, int part) {
-        d = __builtin_amdgcn_mfma_f64_16x16x4f64(a[0], part ? x.y : x.x, d, 0, 0, 0);
-        d = __builtin_amdgcn_mfma_f64_16x16x4f64(a[1], part ? x.x : -x.y, d, 0, 0, 0);
+    template <int NC>
+    __device__ static void fma(acc (&d)[NC], int c0, dvec2 a, dvec2 x, int part) {
+        const double b[K] = {part ? x.y : x.x, part ? x.x : -x.y};
+#pragma unroll
+        for (int e = 0; e < K; e++) {
+            acc& s = d[(c0 + e) % NC];
+            s = __builtin_amdgcn_mfma_f64_16x16x4f64(a[e], b[e], s, 0, 0, 0);
+        }
     }
 };
 
@@ -196,6 +206,19 @@ __device__ __forceinline__ void wave_fence() {
 // 16-byte chunks of LDS a wave needs: 16 rows of A and 8 NT of X, 4 Q chunks
 // and one of padding each.
 constexpr int gemm_wave_chunks(int RT, int NT) { return (16 * RT + 8 * NT) * (4 * kGemmQ + 1); }
+
+// Accumulators per tile.  An MFMA rounds once per product, so one accumulator
+// per wave adds n / 4 products one after the other.  With one column tile every
+// MFMA of a K step has its own: n / 64 (c64) or n / 32 (c128) products and a
+// tree, which is the rounding of the vector tiles' 64 lane sums.  Error of 3
+// sources against 64 bits (c64; c128 against 80), one accumulator and now:
+// n = 330 1.8e-7 and 8.6e-8 (vector tile 9.0e-8), 9990 9.0e-7 and 2.4e-7
+// (3.2e-7); c128 330 3.1e-16 and 1.7e-16 (1.7e-16), 9990 1.6e-15 and 6.2e-16
+// (6.2e-16).  Times are the same within 3 %.
+template <typename T, int NT>
+constexpr int gemm_chains() {
+    return NT == 1 ? kGemmQ * MfmaTile<T>::K : 1;
+}
 
 // The right-hand sides [s0, s0 + 8 NT) of rows [r0, r0 + 16 RT).
 template <typename T, int RT, int NT, bool STREAM>
@@ -219,13 +242,16 @@ __device__ __forceinline__ void gemm_pass(const MvDev& J, int r0, int s0, typena
 #pragma unroll
     for (int k = 0; k < LX; k++)
         gx[k] = (const V*)(glob((const cplx_t<T>*)J.x) + (size_t)n * min(s0 + (64 * k + lane) / CH, J.S - 1));
-    typename M::acc acc[RT][NT];
+    constexpr int NC = gemm_chains<T, NT>();
+    typename M::acc acc[RT][NT][NC];
 #pragma unroll
     for (int t = 0; t < RT; t++)
 #pragma unroll
         for (int u = 0; u < NT; u++)
 #pragma unroll
-            for (int i = 0; i < 4; i++) acc[t][u][i] = 0;
+            for (int c = 0; c < NC; c++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) acc[t][u][c][i] = 0;
     const int nv = n / C;  // 16-byte chunks per row (n is even)
     const int steps = (nv + CH - 1) / CH;
     V a[LA], x[LX];
@@ -259,12 +285,20 @@ __device__ __forceinline__ void gemm_pass(const MvDev& J, int r0, int s0, typena
             for (int u = 0; u < NT; u++) {
                 const V xv = lx[(8 * u + (col >> 1)) * RS + 4 * q + g];
 #pragma unroll
-                for (int t = 0; t < RT; t++) M::fma(acc[t][u], av[t], xv, part);
+                for (int t = 0; t < RT; t++) M::fma(acc[t][u], q * M::K, av[t], xv, part);
             }
         }
         wave_fence();  // the next step's writes stay behind these reads
     }
-    // the waves' tiles, added in wave order (over the operand buffers)
+#pragma unroll
+    for (int t = 0; t < RT; t++)
+#pragma unroll
+        for (int u = 0; u < NT; u++)
+#pragma unroll
+            for (int h = NC / 2; h > 0; h /= 2)
+#pragma unroll
+                for (int c = 0; c < h; c++) acc[t][u][c] += acc[t][u][c + h];
+    // the waves' tiles, added as a tree (over the operand buffers)
     constexpr int TILE = RT * NT * 256;
     T* red = (T*)lds;
     __syncthreads();
@@ -273,12 +307,17 @@ __device__ __forceinline__ void gemm_pass(const MvDev& J, int r0, int s0, typena
 #pragma unroll
         for (int u = 0; u < NT; u++)
 #pragma unroll
-            for (int i = 0; i < 4; i++) red[w * TILE + ((t * NT + u) * 4 + i) * 64 + lane] = acc[t][u][i];
+            for (int i = 0; i < 4; i++) red[w * TILE + ((t * NT + u) * 4 + i) * 64 + lane] = acc[t][u][0][i];
     __syncthreads();
     for (int e = tid; e < TILE; e += 64 * W) {
-        T v = red[e];
+        T p[W];
 #pragma unroll
-        for (int k = 1; k < W; k++) v += red[k * TILE + e];
+        for (int k = 0; k < W; k++) p[k] = red[k * TILE + e];
+#pragma unroll
+        for (int h = W / 2; h > 0; h /= 2)
+#pragma unroll
+            for (int k = 0; k < h; k++) p[k] += p[k + h];
+        T v = p[0];
         const int l = e & 63, i = (e >> 6) & 3, tu = e >> 8, t = tu / NT, u = tu - t * NT;
         const int r = r0 + 16 * t + M::row(l >> 4, i), s = s0 + 8 * u + ((l & 15) >> 1);
         if (r < n && s < J.S) {
@@ -395,7 +434,10 @@ int rows_of_variant(int c, int v) {
 // 12.5, 2910 24 and 45, 4500 51 and 69, 9000 189 and 260, 20000 920 and 982; 8
 // right-hand sides c64 5600 46 and 306, 9648 133 and 511, 16000 304 and 844.
 double tile_weight(int c, int R, int es, long rounds) {
-    if (c >= 2) return R == 1 ? 1.05 : 1.0;  // one 16-row tile reads X twice as often as two
+    // One 16-row tile reads X twice as often as two.  Two c128 tiles with an accumulator per MFMA fill the
+    // registers: where 16 rows do as well they are faster (n = 16000, 8 sources: 592 and 617 us).
+    if (c == 2 && es == 8 && R == 2 && rounds > 1) return 1.1;
+    if (c >= 2) return R == 1 ? 1.05 : 1.0;
     if (c == 0) {
         if (R == 8) return rounds <= 2 ? 1.001 : 1.0;  // r4u2 first where both fill the same rounds
         return R == 1 ? 1.12 : R == 2 ? 1.04 : 1.0;    // x is read R times less often than A

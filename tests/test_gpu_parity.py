@@ -323,6 +323,39 @@ def test_every_matvec_variant_and_autotune(dev):
             assert np.max(np.abs(y - ref)) <= tol * np.abs(ref).max()
 
 
+@pytest.mark.parametrize("c64", [True, False])
+@pytest.mark.parametrize("n,seeds", [(40, 100), (330, 24), (2000, 8)])
+def test_few_source_products_round_like_one_source(dev, c64, n, seeds):
+    """The matrix-core products of 3 to 8 sources round no worse than the
+    vector tile of one: the rounding error (2-norm, over `seeds` Gaussian
+    systems, c64 against 64 bits and c128 against 80) is within 1.1 of it.
+    Both are sqrt(L / 2 + log2 C) in units of the rounding, for C chains of
+    L additions and a tree over them, with L = n / 32, C = 64 for one source
+    and no longer chains for the others; the samples (2000 values and more)
+    give the ratio to 2 %."""
+    import torch
+    dtype = dev.C64 if c64 else dev.C128
+    err = {1: [0.0, 0.0], 3: [0.0, 0.0], 4: [0.0, 0.0], 8: [0.0, 0.0]}
+    g = torch.Generator(device="cuda").manual_seed(n)
+    for _ in range(seeds):
+        A = torch.randn((n, n), dtype=dtype, device="cuda", generator=g)
+        x = torch.randn((8, n), dtype=dtype, device="cuda", generator=g)
+        rows = np.arange(n) if n <= 400 else np.sort(np.random.default_rng(n).choice(n, 200, replace=False))
+        wide = np.complex128 if c64 else np.clongdouble
+        ref = x.cpu().numpy().astype(wide) @ A.cpu().numpy()[rows].astype(wide).T
+        for S, e in err.items():
+            if S == 1:
+                y = torch.cat([dev.matvec(A, x[s:s + 1]) for s in range(3)])
+            else:
+                y = dev.matvec(A, x[:S].contiguous())
+            d = y.cpu().numpy()[:3][:, rows] - ref[:3]
+            e[0] += float(np.sum(np.abs(d) ** 2))
+            e[1] += float(np.sum(np.abs(ref[:3]) ** 2))
+    rel = {S: (a / b) ** 0.5 for S, (a, b) in err.items()}
+    for S in (3, 4, 8):
+        assert rel[S] <= 1.1 * rel[1], rel
+
+
 def test_batched_matvec_autotune(dev):
     """The batched autotuner times the variants of the class of nrhs[0] on one
     launch over several systems (one of another class left out) and leaves a
