@@ -189,6 +189,18 @@ __device__ __forceinline__ double2 csel(bool c, double2 x, double2 y) {
     return make_double2(c ? x.x : y.x, c ? x.y : y.y);
 }
 
+// a / b from inv, a reciprocal of b good to a few units in the last place: the
+// product alone carries the reciprocal's rounding into every entry, one step on
+// the remainder a - q b takes it out (diagonally dominant n = 20: error of the
+// solution 2.14e-16 and 2.04e-16, 2.02e-16 with a division per entry).
+__device__ __forceinline__ double2 cquot(double2 a, double2 b, double2 inv) {
+    double2 q = cmul(a, inv);
+    const double rx = fma(q.y, b.y, fma(-q.x, b.x, a.x)), ry = fma(-q.y, b.x, fma(-q.x, b.y, a.y));
+    q.x = fma(-ry, inv.y, fma(rx, inv.x, q.x));
+    q.y = fma(ry, inv.x, fma(rx, inv.y, q.y));
+    return q;
+}
+
 constexpr int kStripT = 512;  // threads of the strip kernel: 256 registers each
 
 // Rows a thread holds at a strip width (4 registers per entry, about 200 in all).
@@ -354,7 +366,7 @@ __global__ __launch_bounds__(kStripT) void k_lu_strip(double2* __restrict__ A, i
         double2 l[RPT], done[RPT];
 #pragma unroll
         for (int i = 0; i < RPT; i++) {
-            l[i] = cmul(a[i][0], inv);
+            l[i] = cquot(a[i][0], pj, inv);
             done[i] = csel(i > 0 || t > jj, l[i], a[i][0]);  // rows up to j are final
         }
 #pragma unroll
@@ -648,8 +660,11 @@ __global__ __launch_bounds__(kT) void k_lu_permute(const double2* __restrict__ b
 
 // Diagonal block [b0, b0 + nb) of L (unit lower, LOWER) or U (upper, with its
 // diagonal): one wave per right-hand side (grid.x), lane q holds unknown q.  A
-// solved unknown is broadcast and every lane takes its term off: a step is a
+// solved unknown is broadcast and every lane adds its term: a step is a
 // broadcast and one multiply-add, where a wave-wide sum per row took 0.5 us.
+// The terms are summed apart from y and taken off once: off y one by one, each
+// rounds at the size of y (diagonally dominant n = 33: error of the solution
+// 3.5e-16, 2.6e-16 so).
 __device__ __forceinline__ double lane_value(double v, int lane) {
     return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
                             __builtin_amdgcn_readlane(__double2loint(v), lane));
@@ -670,12 +685,15 @@ __global__ __launch_bounds__(kT) void k_lu_diag_solve(const double2* __restrict_
     double2* xs = x + (size_t)blockIdx.x * n + b0;
     double2 y = q < nb ? xs[q] : make_double2(0.0, 0.0);
     const double2 inv = !LOWER && q < nb ? cdiv(make_double2(1.0, 0.0), B[q][q]) : make_double2(1.0, 0.0);
+    double2 t = make_double2(0.0, 0.0);  // this unknown's sum of solved terms
     for (int k = 0; k < nb; k++) {
         const int r = LOWER ? k : nb - 1 - k;
         const double2 b = B[q][r];
-        if (!LOWER && q == r) y = cmul(y, inv);
-        const double2 s = make_double2(lane_value(y.x, r), lane_value(y.y, r));
-        if (q < nb && (LOWER ? q > r : q < r)) y = csub(y, cmul(b, s));
+        double2 v = csub(y, t);
+        if (!LOWER) v = cquot(v, b, inv);
+        const double2 s = make_double2(lane_value(v.x, r), lane_value(v.y, r));
+        if (q == r) y = v;
+        if (q < nb && (LOWER ? q > r : q < r)) cfma(t, b, s);
     }
     if (q < nb) xs[q] = y;
 }

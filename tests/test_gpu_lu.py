@@ -174,3 +174,35 @@ def test_lu_singular_column_inside_a_strip(dev):
     A[:, 531] = 0.0
     with pytest.raises(np.linalg.LinAlgError, match="column 531"):
         dev.lu_solve(dev.to_device(A, dev.C128), dev.to_device(b, dev.C128))
+
+
+@pytest.mark.parametrize("n,seeds", [(20, 100), (33, 60)])
+def test_lu_rounds_like_division_and_dot_products(dev, n, seeds):
+    """The pivot reciprocal and the substitution's order add no error: on
+    diagonally dominant systems, where no pivot growth hides it, the rms error
+    of the solution (against refinement in 80 bits) is within 1.2 of textbook
+    elimination with a division per entry and dot-product substitution; the
+    spread of one system's error is 20 %, so of the rms 2-3 %."""
+    rng = np.random.default_rng(n)
+    ours, book = [], []
+    for _ in range(seeds):
+        A = np.eye(n) + (rng.normal(size=(n, n)) + 1j * rng.normal(size=(n, n))) * (0.4 / (2 * n) ** 0.5)
+        b = rng.normal(size=n) + 1j * rng.normal(size=n)
+        x = np.linalg.solve(A, b).astype(np.clongdouble)
+        for _ in range(2):
+            x += np.linalg.solve(A, (b - A.astype(np.clongdouble) @ x).astype(complex))
+        got = dev.lu_solve(dev.to_device(A, dev.C128), dev.to_device(b[None], dev.C128)).cpu().numpy()[0]
+        LU, y = A.copy(), b.copy()
+        for j in range(n):
+            p = j + np.argmax(np.abs(LU[j:, j]))
+            LU[[j, p]], y[[j, p]] = LU[[p, j]], y[[p, j]]
+            LU[j + 1:, j] /= LU[j, j]
+            LU[j + 1:, j + 1:] -= np.outer(LU[j + 1:, j], LU[j, j + 1:])
+        for i in range(n):
+            y[i] -= LU[i, :i] @ y[:i]
+        for i in reversed(range(n)):
+            y[i] = (y[i] - LU[i, i + 1:] @ y[i + 1:]) / LU[i, i]
+        ours.append(float(np.linalg.norm(got - x) / np.linalg.norm(x)))
+        book.append(float(np.linalg.norm(y - x) / np.linalg.norm(x)))
+    rms = [np.sqrt(np.mean(np.square(e))) for e in (ours, book)]
+    assert rms[0] <= 1.2 * rms[1], rms
