@@ -214,7 +214,7 @@ constexpr int gemm_wave_chunks(int RT, int NT) { return (16 * RT + 8 * NT) * (4 
 // sources against 64 bits (c64; c128 against 80), one accumulator and now:
 // n = 330 1.8e-7 and 8.6e-8 (vector tile 9.0e-8), 9990 9.0e-7 and 2.4e-7
 // (3.2e-7); c128 330 3.1e-16 and 1.7e-16 (1.7e-16), 9990 1.6e-15 and 6.2e-16
-// (6.2e-16).  Times are the same within 3 %.
+// (6.2e-16).
 template <typename T, int NT>
 constexpr int gemm_chains() {
     return NT == 1 ? kGemmQ * MfmaTile<T>::K : 1;
@@ -228,20 +228,21 @@ __device__ __forceinline__ void gemm_pass(const MvDev& J, int r0, int s0, typena
     constexpr int W = kGemmW, Q = kGemmQ, C = M::C, CH = 4 * Q, RS = CH + 1;  // chunks per row and K step; padded row in LDS
     constexpr int LA = RT * Q, LX = NT * Q / 2;            // loads per lane: 16 (or 8 NT) rows x CH chunks / 64
     const int n = J.n;
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = lane >> 4, col = lane & 15, part = col & 1;
     V* la = lds + w * gemm_wave_chunks(RT, NT);
     V* lx = la + 16 * RT * RS;
-    // lane's chunk of load k: id = 64 k + lane, row id / CH, chunk id % CH
-    const V* ga[LA];
-    const V* gx[LX];
+    // lane's chunk of load k: id = 64 k + lane, row id / CH, chunk id % CH, as a byte offset from the pass's
+    // first row and source, whose addresses stay in scalar registers
+    const char* A0 = (const char*)(glob((const cplx_t<T>*)J.A) + (size_t)n * r0);
+    const char* x0 = (const char*)(glob((const cplx_t<T>*)J.x) + (size_t)n * s0);
+    constexpr unsigned ES = sizeof(cplx_t<T>);
+    unsigned oa[LA], ox[LX];
     const int ch = lane % CH;
 #pragma unroll
-    for (int k = 0; k < LA; k++)
-        ga[k] = (const V*)(glob((const cplx_t<T>*)J.A) + (size_t)n * min(r0 + (64 * k + lane) / CH, n - 1));
+    for (int k = 0; k < LA; k++) oa[k] = (unsigned)min((64 * k + lane) / CH, n - 1 - r0) * n * ES + 16 * ch;
 #pragma unroll
-    for (int k = 0; k < LX; k++)
-        gx[k] = (const V*)(glob((const cplx_t<T>*)J.x) + (size_t)n * min(s0 + (64 * k + lane) / CH, J.S - 1));
+    for (int k = 0; k < LX; k++) ox[k] = (unsigned)min((64 * k + lane) / CH, J.S - 1 - s0) * n * ES + 16 * ch;
     constexpr int NC = gemm_chains<T, NT>();
     typename M::acc acc[RT][NT][NC];
 #pragma unroll
@@ -256,17 +257,18 @@ __device__ __forceinline__ void gemm_pass(const MvDev& J, int r0, int s0, typena
     const int steps = (nv + CH - 1) / CH;
     V a[LA], x[LX];
     auto load = [&](int kb) {
-        const int c = kb * CH + ch;
-        const bool in = c < nv;
-        if (STREAM) {
+        const bool in = kb * CH + ch < nv;
+        // Opaque, or the compiler keeps a 64-bit pointer per load: 30 registers more, which leave one
+        // workgroup per CU (30 systems of n = 640, c64, 8 sources: 184 us per iteration, 169 with two).
+        unsigned step = kb * (16 * CH);
+        asm volatile("" : "+s"(step));
 #pragma unroll
-            for (int k = 0; k < LA; k++) a[k] = in ? __builtin_nontemporal_load(ga[k] + c) : V(0);
-        } else {
-#pragma unroll
-            for (int k = 0; k < LA; k++) a[k] = in ? ga[k][c] : V(0);
+        for (int k = 0; k < LA; k++) {
+            const V* p = (const V*)(A0 + (size_t)(oa[k] + step));
+            a[k] = !in ? V(0) : STREAM ? __builtin_nontemporal_load(p) : *p;
         }
 #pragma unroll
-        for (int k = 0; k < LX; k++) x[k] = in ? gx[k][c] : V(0);
+        for (int k = 0; k < LX; k++) x[k] = in ? *(const V*)(x0 + (size_t)(ox[k] + step)) : V(0);
     };
     if (w < steps) load(w);
     for (int kb = w; kb < steps; kb += W) {
@@ -434,10 +436,7 @@ int rows_of_variant(int c, int v) {
 // 12.5, 2910 24 and 45, 4500 51 and 69, 9000 189 and 260, 20000 920 and 982; 8
 // right-hand sides c64 5600 46 and 306, 9648 133 and 511, 16000 304 and 844.
 double tile_weight(int c, int R, int es, long rounds) {
-    // One 16-row tile reads X twice as often as two.  Two c128 tiles with an accumulator per MFMA fill the
-    // registers: where 16 rows do as well they are faster (n = 16000, 8 sources: 592 and 617 us).
-    if (c == 2 && es == 8 && R == 2 && rounds > 1) return 1.1;
-    if (c >= 2) return R == 1 ? 1.05 : 1.0;
+    if (c >= 2) return R == 1 ? 1.05 : 1.0;  // one 16-row tile reads X twice as often as two
     if (c == 0) {
         if (R == 8) return rounds <= 2 ? 1.001 : 1.0;  // r4u2 first where both fill the same rounds
         return R == 1 ? 1.12 : R == 2 ? 1.04 : 1.0;    // x is read R times less often than A
