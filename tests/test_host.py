@@ -103,3 +103,20 @@ def test_serving_arena_first_fit_and_coalescing():
     v = a.view(a.alloc(256), 256, torch.complex128, (4, 4))
     v[:] = 1 + 2j
     assert v.dtype == torch.complex128 and complex(v.sum()) == 16 + 32j
+
+
+@pytest.mark.parametrize("dtype", [0, 1])
+@pytest.mark.parametrize("nrhs,unit", [(1, 32), (2, 16), (8, 64), (16, 64)])
+def test_matvec_tiles_of_a_list_divide_its_blocks(dtype, nrhs, unit):
+    """A batched product splits every block of its work list into tiles by
+    itself: the size rule takes only tiles that divide the block, however many
+    blocks there are; a single system may take any tile."""
+    from miepy_amd import _lib
+    tile = _lib.load().mpa_internal_matvec_tile
+    code = (_lib.MPA_C128, _lib.MPA_C64)[dtype]
+    if nrhs > 2 and code == _lib.MPA_C64:
+        unit = 128
+    used = {tile(code, nrhs, nwork, 0) for nwork in range(1, 6000)}
+    assert all(unit % t == 0 for t in used) and len(used) >= 2
+    if nrhs <= 2:
+        assert any(unit % tile(code, nrhs, 1, n) for n in range(2, 30000, 50))
