@@ -417,3 +417,39 @@ def test_assembly_autotune_variants_match_oracle(dev, oracle):
         assert J >= 1 and ms > 0
         got = dev.assemble(pos, mie, k).cpu().numpy()
         assert np.max(np.abs(got - ref)) <= 1e-13 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("c64", [True, False])
+@pytest.mark.parametrize("S", [1, 2, 8, 16])
+def test_every_matvec_variant_on_a_work_list(dev, c64, S):
+    """A batched launch addresses its rows through work lists, split into tiles
+    that may not divide a list's block: with every tile variant fixed in turn,
+    systems of uneven size (rows not a multiple of the block, one block and
+    less) solved together give what each gives alone at the same tile, bit for
+    bit, and the solutions of the size rule's tile."""
+    import torch
+    import miepy_amd._lib as L
+    lib = L.load()
+    dtype, code, tol = (dev.C64, L.MPA_C64, 1e-5) if c64 else (dev.C128, L.MPA_C128, 1e-11)
+    g = torch.Generator(device="cuda").manual_seed(S)
+    mats, rhs = [], []
+    for n in (6, 30, 130, 334, 610):
+        A = torch.randn((n, n), dtype=dtype, device="cuda", generator=g) * (0.3 / n ** 0.5)
+        mats.append(A + torch.eye(n, dtype=dtype, device="cuda"))
+        rhs.append(torch.randn((S, n), dtype=dtype, device="cuda", generator=g))
+    saved = lib.mpa_matvec_variant(code, S, -1)
+    first, v = None, 0
+    try:
+        while lib.mpa_matvec_variant_name(code, S, v):
+            assert lib.mpa_matvec_variant(code, S, v) == v
+            xs, reps = dev.bicgstab_batched(mats, rhs, tol=tol, maxiter=200)
+            for A, b, x, rep in zip(mats, rhs, xs, reps):
+                x1, rep1 = dev.bicgstab(A, b, tol=tol, maxiter=200)
+                assert rep.converged and rep.iterations == rep1.iterations
+                assert torch.equal(x, x1), lib.mpa_matvec_variant_name(code, S, v).decode()
+            first = first or xs
+            assert all(torch.equal(x, f) for x, f in zip(xs, first))
+            v += 1
+    finally:
+        lib.mpa_matvec_variant(code, S, saved)
+    assert v >= 3
