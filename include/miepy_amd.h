@@ -44,7 +44,7 @@ extern "C" {
 /* runtime options (mpa_set_option / mpa_get_option) */
 #define MPA_OPT_GRAPHS 0 /* 1 (default): the solver loops replay their iterations from a captured
                             HIP graph (one launch per iteration instead of one per kernel) where that
-                            is faster, in batches of many matrix-free systems; 2: always; 0: eager
+                            is faster, in batches of many small FP64 matrix-free systems; 2: always; 0: eager
                             launches.  Results are identical either way.  Graphs are not used while
                             launch timing (mpa_profile_enable) is on. */
 #define MPA_OPT_MATFREE_FP64_KERNEL 1 /* kernel of the FP64 matrix-free product: 0 (default) the FP64

@@ -764,18 +764,29 @@ int read_scalars(const Plan& P, std::vector<Scal>& out, hipStream_t st, bool noa
     return MPA_OK;
 }
 
-// Whether a plan's iterations are replayed from a graph (MPA_OPT_GRAPHS 2:
-// always, 0: never).  A replayed kernel starts about 1 us later than an eager
-// one and the capture costs each solve some 60 us, so eager launches win as
-// long as the host keeps ahead of the GPU: n = 592 33.2 us per iteration
-// replayed and 27.9 eager, a batch of 12 clusters 27.5 and 26.6 ms, 1000
-// spheres matrix-free 9.5 and 9.05 ms.  Many matrix-free systems, each with
-// its own launches, turn that around: 24 clusters 12.3 ms replayed and 13.3
-// eager, 64 clusters 34.2 and 37.0.
-constexpr size_t kGraphMatfree = 16;
-bool graphs_pay(const Plan& P) {
+// Whether iterations are replayed from a graph by default.  A replayed kernel
+// starts about 1 us later than an eager one, the capture costs each solve some
+// 60 us, and a replayed fork to the side stream costs more than an eager one;
+// so eager launches win as long as the host keeps ahead of the GPU.  It falls
+// behind where many FP64 matrix-free systems, each with its own 3 launches per
+// product (complex64 systems share theirs), are all small.  Eager over replayed
+// time of a solve: 12 FP64 systems of up to 10 spheres at lmax 2 1.07, 48 1.08;
+// 24 of up to 60 spheres at lmax 2 1.03; 12 at lmax 3 0.97, of 30 spheres and 8
+// sources 0.95; complex64 with FP64 refinement 12 and 48 of 30 spheres 0.93 and
+// 0.94; FP64 with half the systems stored 0.8 to 0.97.
+constexpr int kReplaySystems = 8;
+constexpr long long kReplayUnknowns = 1024;  // per system, right-hand sides included
+bool replay_pays(int dtype, int stored, int matfree, long long unknowns) {
+    return dtype == MPA_C128 && stored == 0 && matfree >= kReplaySystems && unknowns <= kReplayUnknowns * matfree;
+}
+// MPA_OPT_GRAPHS 2: always, 0: never
+bool use_replay(const Plan& P, int dtype) {
     const int opt = mpa_option(MPA_OPT_GRAPHS);
-    return opt == 2 || (opt != 0 && P.mf_ps.size() >= kGraphMatfree);
+    if (opt == 0 || opt == 2) return opt == 2;
+    const int matfree = (int)P.mf_ps.size();
+    long long unknowns = 0;
+    for (const SysDev& d : P.sys) unknowns += (long long)d.n * d.S;
+    return replay_pays(dtype, (int)P.sys.size() - matfree, matfree, unknowns);
 }
 
 // k BiCGSTAB iterations of a plan recorded once as a HIP graph and replayed.
@@ -829,7 +840,7 @@ int solve_batch(int nsys, const mpa_system* S_, void* scratch, int* iters, doubl
     std::vector<Scal> host;
     long launched = 0;
     IterGraph graph;
-    const bool use_graph = !noalloc && graphs_pay(P) && !mpa_profile_active();
+    const bool use_graph = !noalloc && use_replay(P, dtype) && !mpa_profile_active();
     if (use_graph) {
         rc = capture_iterations<T>(P, k_sync, graph);
         if (rc) return rc;
@@ -1006,6 +1017,11 @@ int mpa_internal_solve_batch(int nsys, const mpa_system* systems, int dtype, voi
 }
 
 extern "C" {
+
+// The default rule of MPA_OPT_GRAPHS (not part of the public interface).
+int mpa_internal_replay_pays(int dtype, int stored, int matfree, long long unknowns) {
+    return replay_pays(dtype, stored, matfree, unknowns) ? 1 : 0;
+}
 
 size_t mpa_system_state_bytes(int n, int nrhs, int dtype) { return state_bytes(n, nrhs, dtype); }
 

@@ -3,6 +3,8 @@ C ABI: every system's result equals its own single-system solve bit for bit
 (the per-system arithmetic and reduction order do not depend on the batch),
 and agrees with the CPU oracle's Eigen-style BiCGSTAB iteration counts."""
 
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -219,6 +221,41 @@ def test_overlapped_product_phases_equal_sequential(dev):
         for a, b in zip(out[key], ref):
             for k in ("p_inc", "C_total", "F"):
                 assert np.array_equal(a[k], b[k]), (key, k)
+
+
+def test_default_replay_equals_eager(dev):
+    """The batches that the default MPA_OPT_GRAPHS replays (8 and more small
+    FP64 matrix-free systems), solved several times with synchronizations
+    between, and a batch beside a stored system, which it does not replay, give
+    the eager launches' results bit for bit."""
+    import torch
+    import miepy_amd._lib as L
+    lib = L.load()
+    systems = [s for s in _systems(dev, seed=8, count=60) if s[3].size <= 1024][:17]
+    assert len(systems) == 17
+    bs = [dev.to_device(b, dev.C128) for *_, b in systems]
+    ops = [dev.ClusterOperator(pos, ms, k, max_rhs=b.shape[0]) for pos, ms, k, b in systems]
+    pos, ms, k, _ = systems[-1]
+    mixed = ops[:-1] + [dev.assemble(pos, ms, k)]
+    assert lib.mpa_get_option(L.MPA_OPT_GRAPHS) == 1
+    assert lib.mpa_internal_replay_pays(L.MPA_C128, 0, 17, ctypes.c_longlong(sum(b.numel() for b in bs)))
+    assert lib.mpa_internal_replay_pays(L.MPA_C128, 0, 8, ctypes.c_longlong(sum(b.numel() for b in bs[:8])))
+    out = {}
+    try:
+        for mode in (1, 0):
+            assert lib.mpa_set_option(L.MPA_OPT_GRAPHS, mode) == 0
+            out[mode] = []
+            for _ in range(3 if mode else 1):
+                for A, b in ((ops, bs), (ops[:8], bs[:8]), (mixed, bs)):
+                    xs, reps = dev.bicgstab_batched(A, b, tol=1e-10, maxiter=2000, add_identity=True)
+                    torch.cuda.synchronize()
+                    assert all(r.converged for r in reps)
+                    out[mode] += list(zip(xs, [r.iterations for r in reps]))
+    finally:
+        lib.mpa_set_option(L.MPA_OPT_GRAPHS, 1)
+    for q, (x, it) in enumerate(out[1]):
+        xe, ie = out[0][q % len(out[0])]
+        assert it == ie and torch.equal(x, xe)
 
 
 def test_batched_assembly_equals_single(dev):

@@ -3,6 +3,8 @@ reference's Python host (plane-wave mode tables, workloads, backend
 registry, serving arena).  CPU only; the Mie coefficients and per-particle
 p_src run on the device (tests/test_gpu_inputs.py)."""
 
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -120,3 +122,21 @@ def test_matvec_tiles_of_a_list_divide_its_blocks(dtype, nrhs, unit):
     assert all(unit % t == 0 for t in used) and len(used) >= 2
     if nrhs <= 2:
         assert any(unit % tile(code, nrhs, 1, n) for n in range(2, 30000, 50))
+
+
+def test_graph_replay_rule():
+    """By default iterations are replayed from a graph only where the launches
+    of many small FP64 matrix-free systems outrun the host: not for complex64
+    (its systems share launches), not beside stored systems (the fork to the
+    side stream is dearer in a graph), not for few or large systems."""
+    from miepy_amd import _lib
+    pays = _lib.load().mpa_internal_replay_pays
+    pays.argtypes = [ctypes.c_int] * 3 + [ctypes.c_longlong]
+    small, large = 160, 5400  # unknowns: 10 spheres at lmax 2; 30 at lmax 3 with 6 sources
+    for count in (8, 12, 24, 96):
+        assert pays(_lib.MPA_C128, 0, count, count * small)
+        assert not pays(_lib.MPA_C128, 0, count, count * large)
+        assert not pays(_lib.MPA_C64, 0, count, count * small)
+        assert not pays(_lib.MPA_C128, 1, count, (count + 1) * small)
+    assert not pays(_lib.MPA_C128, 0, 7, 7 * small)
+    assert not pays(_lib.MPA_C128, 5, 0, 5 * small)
