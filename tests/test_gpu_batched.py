@@ -124,7 +124,7 @@ def test_cluster_batch_matches_single_clusters(dev):
 
 
 def test_graph_replay_equals_eager(dev):
-    """Iterations replayed from captured HIP graphs (the default) give the
+    """Iterations replayed from captured HIP graphs (MPA_OPT_GRAPHS 2) give the
     eager launches' results bit for bit, for single and batched solves,
     stored and matrix-free operators, c128 and c64, one or several
     iterations per graph; each solve replays its graph many times with host
@@ -152,8 +152,9 @@ def test_graph_replay_equals_eager(dev):
         out.append((x.cpu().numpy(), rep.iterations))
         return out
 
-    graphed = run()
     try:
+        assert lib.mpa_set_option(L.MPA_OPT_GRAPHS, 2) == 0
+        graphed = run()
         assert lib.mpa_set_option(L.MPA_OPT_GRAPHS, 0) == 0
         eager = run()
     finally:
@@ -191,7 +192,8 @@ def test_overlapped_product_phases_equal_sequential(dev):
     """MPA_OPT_OVERLAP: the batched GEMM over the stored matrices on the side
     stream beside the matrix-free products gives the same solve, bit for bit,
     as the two one after the other, with the iterations replayed from HIP
-    graphs (the fork and join captured as parallel branches) and eagerly."""
+    graphs (MPA_OPT_GRAPHS 2: the fork and join captured as parallel branches)
+    and eagerly."""
     import miepy_amd._lib as L
     from miepy_amd.batch import ClusterBatch
     from miepy_amd.workloads import batch256
@@ -204,7 +206,7 @@ def test_overlapped_product_phases_equal_sequential(dev):
     saved = (lib.mpa_get_option(L.MPA_OPT_OVERLAP), lib.mpa_get_option(L.MPA_OPT_GRAPHS))
     out = {}
     try:
-        for overlap, graphs in ((0, 1), (1, 1), (1, 0)):
+        for overlap, graphs in ((0, 2), (1, 2), (1, 0)):
             lib.mpa_set_option(L.MPA_OPT_OVERLAP, overlap)
             lib.mpa_set_option(L.MPA_OPT_GRAPHS, graphs)
             B = ClusterBatch(ws, precision="mixed_matfree", matfree_min_n=1500)
@@ -216,8 +218,8 @@ def test_overlapped_product_phases_equal_sequential(dev):
     finally:
         lib.mpa_set_option(L.MPA_OPT_OVERLAP, saved[0])
         lib.mpa_set_option(L.MPA_OPT_GRAPHS, saved[1])
-    ref = out[(0, 1)]
-    for key in ((1, 1), (1, 0)):
+    ref = out[(0, 2)]
+    for key in ((1, 2), (1, 0)):
         for a, b in zip(out[key], ref):
             for k in ("p_inc", "C_total", "F"):
                 assert np.array_equal(a[k], b[k]), (key, k)
@@ -322,7 +324,8 @@ def test_solo_small_system_equals_batch_with_a_large_one(dev, c64):
 def test_forced_graph_replay_equals_eager(dev, sync_every):
     """MPA_OPT_GRAPHS 2 replays every solve from graphs, whatever its size:
     stored and matrix-free systems below and above 4096 unknowns give the
-    eager launches' results bit for bit."""
+    eager launches' results bit for bit, apart and in one batch (whose stored
+    products are captured on the side stream)."""
     import torch
     import miepy_amd._lib as L
     lib = L.load()
@@ -340,8 +343,9 @@ def test_forced_graph_replay_equals_eager(dev, sync_every):
         for mode in (2, 0):
             assert lib.mpa_set_option(L.MPA_OPT_GRAPHS, mode) == 0
             out[mode] = []
-            for ms, rhs in ((mats, bs), (mats + [big], bs + [b_big]), (ops, bs)):
-                xs, reps = dev.bicgstab_batched(ms, rhs, tol=1e-10, maxiter=500, sync_every=sync_every)
+            for ms, rhs in ((mats, bs), (mats + [big], bs + [b_big]), (ops, bs), (ops + [big], bs + [b_big])):
+                xs, reps = dev.bicgstab_batched(ms, rhs, tol=1e-10, maxiter=500, sync_every=sync_every,
+                                                add_identity=isinstance(ms[0], dev.ClusterOperator))
                 out[mode] += list(zip(xs, [r.iterations for r in reps]))
     finally:
         lib.mpa_set_option(L.MPA_OPT_GRAPHS, saved)
