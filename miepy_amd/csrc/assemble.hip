@@ -261,17 +261,20 @@ int launch_assembly(int N, int lmax, const double* positions, const double* mie,
 // its particle's T-matrix on the FP64 matrix cores, as a real product: K
 // position 2q + odd holds Re or Im of X[.][q], real column 2c + part of the
 // right operand Re or Im of the product (Re T, -Im T / Im T, Re T).  A
-// workgroup owns one column block and kApplyRows rows: Tm_j stays in LDS as
-// the right operand, each wave takes 16 rows at a time through its own part of
-// LDS (coalesced in, operand layout out) and writes their products back; the
-// identity is added on the diagonal blocks (which are zero before the
-// product).  110 particles at lmax 3 (174 MB): 187 us with one thread per
-// entry, which read two LDS values per multiply-add, 96 us so.
+// workgroup owns one column block and a run of rows: its four waves split the
+// output columns (up to lmax 2, where one or two column tiles are all there
+// are, also the rows) and keep their part of Tm_j in registers as the right
+// operand, so that LDS holds only the rows at hand, double-buffered, and 16
+// rows cost a wave a quarter of their products.  The products are written
+// from the result registers (8 complex runs of a row); the identity is added
+// on the diagonal blocks (which are zero before the product).  us of the
+// launch with one thread per entry, with Tm_j in LDS (lmax 6: through the
+// caches) and each wave 16 rows of its own, and so: lmax 3, 10 and 120
+// particles 8.6, 19.9, 4.1 and 219, 111, 86; lmax 4, 3 and 80 particles 13.5,
+// 28.6, 5.1 and 389, 218, 163; lmax 5, 30 particles 184, 229, 81; lmax 6, 1 and
+// 50 particles 50, 160, 12 and 1243, 2709, 371 (48 TFLOP/s of FP64 MFMA).
 
 typedef double ad4 __attribute__((ext_vector_type(4)));
-
-constexpr int kApplyRows = 256;  // rows of a workgroup
-constexpr int kApplyWaves = kThreads / 64;
 
 template <typename OutT>
 __device__ inline double2 load_c(const OutT* p);
@@ -285,107 +288,118 @@ __device__ inline double2 load_c<float2>(const float2* p) {
     return make_double2(v.x, v.y);
 }
 
-// LDS: Tm_j [bs][bs + 1] (up to lmax 5; read through the caches above), then per wave 16 rows of X [bs + 1]
+template <int LMAX>
+struct ApplyTile {
+    static constexpr int bs = 2 * LMAX * (LMAX + 2);
+    static constexpr int NT = (bs + 7) / 8;                     // tiles of 8 complex columns
+    static constexpr int WC = NT < 4 ? NT : 4, WR = 4 / WC;     // waves over columns and over rows
+    static constexpr int TW = (NT + WC - 1) / WC;               // column tiles per wave
+    static constexpr int rows = 16 * WR;                        // rows of a step
+};
+
+__device__ __forceinline__ void store_part(double2* p, int part, double v) { ((double*)p)[part] = v; }
+__device__ __forceinline__ void store_part(float2* p, int part, double v) { ((float*)p)[part] = (float)v; }
+
+// Rows [blockIdx.x % nrowblocks * rows, ...) of column block blockIdx.x / nrowblocks; rows a multiple of ApplyTile::rows.
 template <typename OutT, int LMAX>
-__global__ __launch_bounds__(kThreads) void k_apply_tmatrix(int N, int nrowblocks, const double2* __restrict__ tm,
-                                                             int add_identity, OutT* __restrict__ out) {
-    constexpr int bs = 2 * LMAX * (LMAX + 2), ls = bs + 1, NT = (bs + 7) / 8;
-    constexpr bool staged = LMAX <= 5;
-    __shared__ double2 X_[kApplyWaves * 16 * ls];
-    __shared__ double2 T_[staged ? bs * ls : 1];
+__global__ __launch_bounds__(kThreads, 1) void k_apply_tmatrix(int N, int nrowblocks, int rows,
+                                                               const double2* __restrict__ tm, int add_identity,
+                                                               OutT* __restrict__ out) {
+    using A = ApplyTile<LMAX>;
+    constexpr int bs = A::bs, ls = bs + 1, TW = A::TW, TR = A::rows, total = TR * bs;
+    constexpr int LD = (total + kThreads - 1) / kThreads;
+    __shared__ double2 X_[2][TR * ls];
     const int j = blockIdx.x / nrowblocks;
-    const int r0 = (blockIdx.x % nrowblocks) * kApplyRows;
+    const int r0 = (blockIdx.x % nrowblocks) * rows;
     const size_t n = (size_t)bs * N;
-    const int nr = (int)min((size_t)kApplyRows, n - r0);
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, g = lane >> 4, col = lane & 15;
-    const int part = col & 1, odd = g & 1;
-    double2* X = X_ + w * 16 * ls;
-    const double2* tmj = tm + (size_t)j * bs * bs;
-    if (staged) {
-        for (int u = threadIdx.x; u < bs * bs; u += kThreads) T_[(u / bs) * ls + u % bs] = tmj[u];
-        __syncthreads();
-    }
+    const int nr = (int)min((size_t)rows, n - r0);
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wc = w % A::WC, wr = w / A::WC, g = lane >> 4, col = lane & 15, part = col & 1, odd = g & 1;
+    const double* tmj = (const double*)(tm + (size_t)j * bs * bs);
+    // 4 real K positions per step: complex q = 2 s, 2 s + 1 (bs is even)
+    double b[bs / 2][TW];
+#pragma unroll
+    for (int s = 0; s < bs / 2; s++)
+#pragma unroll
+        for (int e = 0; e < TW; e++) {
+            const int c = min(8 * (wc + A::WC * e) + (col >> 1), bs - 1);
+            const double u = tmj[2 * ((2 * s + (g >> 1)) * bs + c) + (odd ^ part)];
+            b[s][e] = odd && !part ? -u : u;
+        }
     OutT* block = out + (size_t)r0 * n + (size_t)j * bs;
-    constexpr int total = 16 * bs;
-    // the next 16 rows are read while the current ones are multiplied
-    constexpr int LD = total / 64 + (total % 64 ? 1 : 0);
-    double2 v[LD];
+    double2 v[LD];  // the next step's rows, read while the current ones are multiplied
     auto load = [&](int t0) {
 #pragma unroll
         for (int e = 0; e < LD; e++) {
-            const int u = min(64 * e + lane, total - 1), rr = u / bs, c = u - rr * bs;
+            const int u = min((int)threadIdx.x + kThreads * e, total - 1), rr = u / bs, c = u - rr * bs;
             v[e] = load_c<OutT>(block + (size_t)min(t0 + rr, nr - 1) * n + c);
         }
     };
-    if (w * 16 < nr) load(w * 16);
-    for (int t0 = w * 16; t0 < nr; t0 += 16 * kApplyWaves) {
+    load(0);
+    for (int t0 = 0, buf = 0; t0 < nr; t0 += TR, buf ^= 1) {
+        double2* X = X_[buf];
 #pragma unroll
         for (int e = 0; e < LD; e++) {
-            const int u = 64 * e + lane, rr = u / bs, c = u - rr * bs;
+            const int u = (int)threadIdx.x + kThreads * e, rr = u / bs, c = u - rr * bs;
             if (u < total) X[rr * ls + c] = v[e];
         }
-        if (t0 + 16 * kApplyWaves < nr) load(t0 + 16 * kApplyWaves);
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        ad4 acc[NT];
+        __syncthreads();  // every column of these rows is read before any is written back
+        if (t0 + TR < nr) load(t0 + TR);
+        ad4 acc[TW];
 #pragma unroll
-        for (int t = 0; t < NT; t++)
+        for (int e = 0; e < TW; e++)
 #pragma unroll
-            for (int q = 0; q < 4; q++) acc[t][q] = 0.0;
-        for (int s = 0; s < bs / 2; s++) {  // 4 real K positions: complex q = 2 s, 2 s + 1 (bs is even)
-            const int q = 2 * s + (g >> 1);
-            const double2 xv = X[col * ls + q];
-            const double a = odd ? xv.y : xv.x;
+            for (int q = 0; q < 4; q++) acc[e][q] = 0.0;
+        const double* Xa = (const double*)(X + (16 * wr + col) * ls + (g >> 1)) + odd;
 #pragma unroll
-            for (int t = 0; t < NT; t++) {
-                const int c = min(8 * t + (col >> 1), bs - 1);
-                const double2 u = staged ? T_[q * ls + c] : tmj[q * bs + c];
-                const double b = odd ? (part ? u.x : -u.y) : (part ? u.y : u.x);
-                acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc[t], 0, 0, 0);
+        for (int s = 0; s < bs / 2; s++) {
+            const double a = Xa[4 * s];
+#pragma unroll
+            for (int e = 0; e < TW; e++) acc[e] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b[s][e], acc[e], 0, 0, 0);
+        }
+#pragma unroll
+        for (int e = 0; e < TW; e++) {
+            const int c = 8 * (wc + A::WC * e) + (col >> 1);
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int r = t0 + 16 * wr + 4 * q + g;
+                double x = acc[e][q];
+                if (add_identity && part == 0 && (size_t)(r0 + r) == (size_t)j * bs + c) x += 1.0;
+                if (r < nr && c < bs) store_part(block + (size_t)r * n + c, part, x);
             }
         }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        double* Xd = (double*)X;
-#pragma unroll
-        for (int t = 0; t < NT; t++) {
-            const int c = 8 * t + (col >> 1);
-            if (c < bs)
-#pragma unroll
-                for (int q = 0; q < 4; q++) Xd[2 * ((4 * q + g) * ls + c) + part] = acc[t][q];
-        }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        for (int u = lane; u < total; u += 64) {
-            const int rr = u / bs, c = u - rr * bs;
-            if (t0 + rr >= nr) continue;
-            double2 v = X[rr * ls + c];
-            if (add_identity && (size_t)(r0 + t0 + rr) == (size_t)j * bs + c) v.x += 1.0;
-            store<OutT>(block + (size_t)(t0 + rr) * n + c, v);
-        }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
     }
 }
 
-template <typename OutT>
-int launch_apply_tmatrix(int N, int lmax, const double* tmatrix, int add_identity, OutT* out, hipStream_t s) {
-    const int bs = 2 * lmax_to_rmax(lmax);
-    const long long n = (long long)bs * N;
-    const int nrb = (int)((n + kApplyRows - 1) / kApplyRows);
-    const long long nblocks = (long long)N * nrb;
+template <typename OutT, int LMAX>
+int launch_apply(int N, const double* tmatrix, int add_identity, OutT* out, hipStream_t s) {
+    using A = ApplyTile<LMAX>;
+    const long long n = (long long)A::bs * N, steps = (n + A::rows - 1) / A::rows;
+    // Rows of a workgroup: about 32 steps, which hide the read of Tm_j, and as many workgroups as fill a whole
+    // number of rounds over the CUs (two per CU up to lmax 4, whose registers allow them).
+    const long long slots = LMAX <= 4 ? 512 : 256, rounds = (N * steps + slots * 32 - 1) / (slots * 32);
+    const long long runs = std::max(1LL, slots * rounds / N), per = (steps + runs - 1) / runs;
+    const long long nrb = (steps + per - 1) / per, nblocks = N * nrb;
     if (nblocks > 0x7fffffffLL) {
         mpa_set_error("particle_aggregate_tmatrix: N=%d too large for one launch", N);
         return MPA_ERR_ARG;
     }
-#define MPA_APPLY(L_)                                                                                               \
-    if (lmax == L_)                                                                                                 \
-        hipLaunchKernelGGL((k_apply_tmatrix<OutT, L_>), dim3((unsigned)nblocks), dim3(kThreads), 0, s, N, nrb,      \
-                           (const double2*)tmatrix, add_identity, out);
-    MPA_APPLY(1) MPA_APPLY(2) MPA_APPLY(3) MPA_APPLY(4) MPA_APPLY(5) MPA_APPLY(6)
-#undef MPA_APPLY
+    hipLaunchKernelGGL((k_apply_tmatrix<OutT, LMAX>), dim3((unsigned)nblocks), dim3(kThreads), 0, s, N, (int)nrb,
+                       (int)per * A::rows, (const double2*)tmatrix, add_identity, out);
     MPA_LAUNCH_CHECK();
     return MPA_OK;
+}
+
+template <typename OutT>
+int launch_apply_tmatrix(int N, int lmax, const double* tmatrix, int add_identity, OutT* out, hipStream_t s) {
+    switch (lmax) {
+        case 1: return launch_apply<OutT, 1>(N, tmatrix, add_identity, out, s);
+        case 2: return launch_apply<OutT, 2>(N, tmatrix, add_identity, out, s);
+        case 3: return launch_apply<OutT, 3>(N, tmatrix, add_identity, out, s);
+        case 4: return launch_apply<OutT, 4>(N, tmatrix, add_identity, out, s);
+        case 5: return launch_apply<OutT, 5>(N, tmatrix, add_identity, out, s);
+        default: return launch_apply<OutT, 6>(N, tmatrix, add_identity, out, s);
+    }
 }
 
 }  // namespace

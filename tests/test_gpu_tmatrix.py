@@ -130,11 +130,12 @@ def test_cluster_dense_tmatrices_match_oracle_lu(dev, oracle, mode):
     assert np.linalg.norm(cl.p_scat - p_scat) <= 1e-9 * np.linalg.norm(p_scat)
 
 
-@pytest.mark.parametrize("N,lmax", [(1, 1), (43, 1), (17, 2), (18, 3), (6, 4), (4, 5), (3, 6)])
+@pytest.mark.parametrize("N,lmax", [(1, 1), (43, 1), (17, 2), (18, 3), (6, 4), (4, 5), (3, 6),
+                                    (80, 1), (35, 2), (1, 3), (23, 4), (12, 5), (1, 6), (9, 6)])
 def test_particle_aggregate_row_blocks(dev, oracle, N, lmax):
-    """The T-matrix product at row counts below, at and above one workgroup's
-    256 rows and with a partial last group of 16, every order up to 6 (6: the
-    T-matrix is read past LDS): the bars of the oracle test above."""
+    """The T-matrix product at one and several steps of 64, 32 and 16 rows per
+    workgroup, whole and partial, for every order up to 6: the bars of the
+    oracle test above."""
     pos, rng = _geometry(N, 90 + N)
     k = 2 * np.pi / (600 * nm)
     tm = _random_tmatrices(rng, N, lmax)
