@@ -19,6 +19,7 @@
 // Cext[a][n-1] = f sum_m Re(conj(p_src[a][r]) p_cluster[a][r]),
 // Cabs = Cext - Cscat.
 
+#include <algorithm>
 #include <cmath>
 
 #include "translation.hpp"
@@ -51,7 +52,7 @@ __global__ __launch_bounds__(kCT) void k_cluster_coef(int N, int L, int lmax_in,
                                                       const double* __restrict__ pos, double ox, double oy, double oz,
                                                       const double2* __restrict__ p_scat,
                                                       const double2* __restrict__ mie, double origin_tol, double k,
-                                                      TabDev tab, double2* __restrict__ part) {
+                                                      TabDev tab, double2* __restrict__ part, int y0) {
     extern __shared__ double2 lds[];  // XA, XB [rmax_out][rmax_in]
     __shared__ double2 HL[kCoefGroup][kCoefHL];
     __shared__ double2 eph[kCoefGroup][2 * MPA_LMAX_MAX + 1];
@@ -62,9 +63,9 @@ __global__ __launch_bounds__(kCT) void k_cluster_coef(int N, int L, int lmax_in,
     int us[kCoefOut], ur[kCoefOut];  // this thread's outputs (s, r); s < 0: none
 #pragma unroll
     for (int e = 0; e < kCoefOut; e++) {
-        const int u = ((int)blockIdx.y * kCoefOut + e) * kCT + threadIdx.x;
-        us[e] = u < total ? u / rmax_out : -1;
-        ur[e] = u < total ? u % rmax_out : 0;
+        const long long u = ((long long)(y0 + (int)blockIdx.y) * kCoefOut + e) * kCT + threadIdx.x;
+        us[e] = u < total ? (int)u / rmax_out : -1;
+        ur[e] = u < total ? (int)u % rmax_out : 0;
         acc0[e] = acc1[e] = make_double2(0, 0);
     }
     // One test for both uses: special functions are formed for exactly the
@@ -139,10 +140,12 @@ void launch_cluster_coef(int N, int L, int lmax_in, int lmax_out, int S, const d
                          const TabDev& tab, double2* part, hipStream_t st) {
     const int rmax_in = lmax_to_rmax(lmax_in), rmax_out = lmax_to_rmax(lmax_out);
     const long long total = (long long)S * rmax_out;
-    const unsigned gy = (unsigned)((total + kCT * kCoefOut - 1) / (kCT * kCoefOut));
+    const long long blocks = (total + kCT * kCoefOut - 1) / (kCT * kCoefOut);
     const size_t lds = 2 * sizeof(double2) * (size_t)rmax_in * rmax_out;
-    hipLaunchKernelGGL(k_cluster_coef, dim3(chunks_for(N), gy), dim3(kCT), lds, st, N, L, lmax_in, lmax_out, S, pos,
-                       ox, oy, oz, p_scat, mie, origin_tol, k, tab, part);
+    for (long long y0 = 0; y0 < blocks; y0 += 65535)  // a grid's y holds no more (1.4e6 right-hand sides of order 6)
+        hipLaunchKernelGGL(k_cluster_coef, dim3(chunks_for(N), (unsigned)std::min(65535LL, blocks - y0)), dim3(kCT), lds,
+                           st, N, L, lmax_in, lmax_out, S, pos, ox, oy, oz, p_scat, mie, origin_tol, k, tab, part,
+                           (int)y0);
 }
 
 // (A, B) = the translation coefficients of tuples (m, n, u, v) for the

@@ -85,6 +85,22 @@ def test_positions_without_a_distance_give_nan(dev, coord, tiny, N, at):
     assert np.isfinite(T).all() if tiny else np.isnan(T).all()
 
 
+def test_more_right_hand_sides_than_a_grid_holds(dev):
+    """1.4e6 right-hand sides of order 6 are 65625 blocks of outputs, more than
+    a grid's y dimension: every one is formed (their inputs repeat with a
+    period of 7, so the outputs do, bit for bit)."""
+    import torch
+    S = 1_400_000
+    g = torch.Generator(device="cuda").manual_seed(1)
+    p7 = torch.randn((7, 1, 2, 3), dtype=dev.C128, device="cuda", generator=g)
+    p = p7.repeat(S // 7, 1, 1, 1)
+    pos = np.array([[0.7, -0.4, 0.9]])
+    ref = dev.cluster_coefficients(pos, p7, 6.0, np.zeros(3), 6)
+    got = dev.cluster_coefficients(pos, p, 6.0, np.zeros(3), 6)
+    assert torch.isfinite(torch.view_as_real(ref)).all()
+    assert (got.reshape(S // 7, 7, 2, 48) == ref).all()
+
+
 def test_cluster_cross_sections_match_oracle(dev, oracle):
     rng = np.random.default_rng(5)
     for lmax in (1, 3, 6):
