@@ -124,7 +124,10 @@ int mpa_autotune_matvec(int n, int nrhs, int dtype, const void* A, const void* x
 int mpa_autotune_matvec_batched(int count, const int* n, const int* nrhs, int dtype, const void* const* A,
                                 const void* const* x, void* const* y, int reps, int* variant_out, double* ms_out,
                                 void* stream);
-/* Variant in use for (dtype, class of nrhs); set_to >= 0 selects one. */
+/* Variant in use for (dtype, class of nrhs); set_to >= 0 selects one (an id past
+ * the last one leaves it as it is).  0, the default, lets every launch choose by
+ * its size; the others fix a tile.  Ids belong to one version of the library:
+ * look a tile up by its name. */
 int mpa_matvec_variant(int dtype, int nrhs, int set_to);
 const char* mpa_matvec_variant_name(int dtype, int nrhs, int variant);
 
