@@ -366,7 +366,9 @@ __global__ __launch_bounds__(kStripT) void k_lu_strip(double2* __restrict__ A, i
         double2 l[RPT], done[RPT];
 #pragma unroll
         for (int i = 0; i < RPT; i++) {
-            l[i] = cquot(a[i][0], pj, inv);
+            // More rows per thread: the remainder step would cost 1.3 % of a solve (n = 2910), whose error the
+            // longer sums decide (3.7e-15 and 3.8e-15 without and with it).
+            l[i] = W == 16 ? cquot(a[i][0], pj, inv) : cmul(a[i][0], inv);
             done[i] = csel(i > 0 || t > jj, l[i], a[i][0]);  // rows up to j are final
         }
 #pragma unroll
