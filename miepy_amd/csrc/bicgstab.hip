@@ -300,8 +300,9 @@ __global__ __launch_bounds__(kThreads) void k_commit_p(const SysDev* __restrict_
 // thread t of group g, a group is summed by wave and then over its 4 waves, the
 // G group sums as reduce_partials does.  So a system's iterates do not depend
 // on which kernels its batch uses.  us per iteration, products included, one
-// source: n = 592 40.8 -> 34.7, n = 1800 55.2 -> 46.7; at n = 4500 one CU's
-// bandwidth takes the gain back (133.7 and 134.6, two passes).
+// source, five vector launches and two: n = 592 57 and 36, n = 1800 58 and 48,
+// n = 4096 128 and 125; beyond, one CU's bandwidth takes the gain back (n = 4500
+// in two passes 136 either way).
 constexpr int kHalfT = 1024;      // threads: 4 groups of 256
 constexpr int kHalfMaxN = 4096;   // 4 groups of 1024 elements
 

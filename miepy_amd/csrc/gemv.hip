@@ -2,13 +2,14 @@
 // autotuner and the C ABI.  Replaces the OpenMP row-block GEMV of
 // cpp/src/interactions.cpp:62-95 (and the products inside Eigen's BiCGSTAB).
 //
-// The system matrix is streamed from HBM exactly once per pass with 16-byte
-// nontemporal loads (the matrix is not reused within a call, so it is kept
-// out of the caches that hold x).  Vector-ALU tiles: each wave of a
-// workgroup owns R consecutive rows of one system and runs along the full
-// rows with U chunks per lane in flight; the x chunk loaded for a column is
-// reused for the R rows and for up to SG right-hand sides held in registers.
-// Jobs whose system has converged for all right-hand sides return before
+// The system matrix is read from HBM once per pass in 16-byte loads.  It is not
+// reused within a call, so these are nontemporal and leave the caches to x,
+// but for matrix-core tiles over rows that are no whole 128-byte lines
+// (gemm_rows).  Vector-ALU tiles (one pass): each wave of a workgroup owns R
+// consecutive rows of one system and runs along the full rows with U chunks
+// per lane in flight; the x chunk loaded for a column is reused for the R rows
+// and for up to SG right-hand sides held in registers.  Matrix-core tiles: 8
+// right-hand sides per pass up to 8 of them, 16 beyond.  Jobs whose system has converged for all right-hand sides return before
 // touching the matrix.
 
 #include <vector>

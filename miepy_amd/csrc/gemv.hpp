@@ -1,11 +1,12 @@
 // Batched complex matvec y = (I +) A x over many systems, S RHS each.
 //
-// The system matrix is streamed from HBM exactly once per call (per pass of 16
-// right-hand sides) with 16-byte nontemporal loads: it is not reused within a
-// call, so it is kept out of the caches that hold x.  One or two right-hand
-// sides run on the vector units, a wave owning R consecutive rows; three and
-// more run on the matrix cores, a workgroup owning 16 or 32 rows whose columns
-// its waves split.  Jobs whose system has converged for all right-hand sides
+// The system matrix is read from HBM once per pass: one pass for up to 8
+// right-hand sides, one per 16 beyond.  It is not reused within a call, so it is
+// streamed past the caches, which hold x (not by matrix-core tiles over rows
+// that are no whole 128-byte lines).  One or two right-hand sides run on the
+// vector units, a wave owning R consecutive rows; three and more run on the
+// matrix cores, a workgroup owning 16 or 32 rows whose columns its waves split.
+// Jobs whose system has converged for all right-hand sides
 // return before touching the matrix.
 #pragma once
 

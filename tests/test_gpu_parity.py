@@ -77,9 +77,9 @@ def test_single_particle_and_aligned_pairs(dev, oracle):
 
 @pytest.mark.parametrize("S", [1, 2, 3, 5, 8, 11, 16, 21])
 def test_matvec(dev, S):
-    """Every tile class: vector-ALU tiles (S <= 4) and the matrix-core GEMM
-    (S >= 5, 16 RHS per pass, K steps of 32 columns with a ragged tail,
-    partial row blocks)."""
+    """Every tile class: vector-ALU tiles (S <= 2) and the matrix-core GEMM
+    (S <= 8 in one pass, 16 RHS per pass beyond, K steps of 32 complex64 or 16
+    complex128 columns with a ragged tail, partial row blocks)."""
     rng = np.random.default_rng(S)
     for n in (30, 64, 130, 600, 1000):
         A = rng.normal(size=(n, n)) + 1j * rng.normal(size=(n, n))
