@@ -435,7 +435,7 @@ int rows_of_variant(int c, int v) {
 // 27 sizes tried from 592 to 30000 rows.  us per product, this rule and the
 // fixed r8u2 / 128-row tiles that served every size before: n = 592 c128 7.3 and
 // 12.5, 2910 24 and 45, 4500 51 and 69, 9000 189 and 260, 20000 920 and 982; 8
-// right-hand sides c64 5600 46 and 306, 9648 133 and 511, 16000 304 and 844.
+// right-hand sides c64 5600 46 and 306, 9648 132 and 511, 16000 301 and 844.
 double tile_weight(int c, int R, int es, long rounds) {
     if (c >= 2) return R == 1 ? 1.05 : 1.0;  // one 16-row tile reads X twice as often as two
     if (c == 0) {
@@ -449,8 +449,9 @@ double tile_weight(int c, int R, int es, long rounds) {
 // block: rows of a work-list block, 0 for one job.  A list splits every block by
 // itself, so there only tiles that divide the block are counted rightly, and the
 // others leave part-filled workgroups: 12 systems of n = 2500 (c128, 1 source;
-// 948 blocks of 32) ran 24-row tiles, 24 + 8 rows per block, at 863 us per
-// BiCGSTAB iteration, 785 us with the 32 rows that serve them now.
+// 948 blocks of 32) ran 24-row tiles, 24 + 8 rows per block, at 866 us per
+// BiCGSTAB iteration; 785 us in 32-row tiles, 710 us in the 8-row ones that
+// fill the rounds best.
 int auto_variant(int c, long rows, int es, int block) {
     constexpr long kCus = 256;
     int best = 1;
